@@ -186,7 +186,7 @@ struct dalm_ctx {
     int precision = DALM_FP64;
     hipStream_t stream = nullptr;
     int grid = 0;   // blocks for the cell kernels (tile loop)
-    int ncu = 256;  // compute units of an MI355X (sizes the one-block-per-CU fused kernels)
+    int ncu = 256;  // compute units (sizes the one-block-per-CU fused kernels and the resident solvers)
     int sgrid = 0;  // blocks of the column-streaming stencil kernels (= d.nunits)
 
     // mesh (device)
@@ -246,6 +246,13 @@ struct dalm_ctx {
     SolveState* h_solve = nullptr; // pinned host mirror
     StepScalars* scal = nullptr;   // device
     StepScalars* h_scal = nullptr; // pinned host
+
+    // exchange slots of the resident solvers (resident.h), allocated on first use; dirty:
+    // to be emptied before the next launch; off: this context does without them
+    void* res_ring = nullptr;
+    int* res_abort = nullptr;
+    bool res_dirty = true, res_off = false;
+    int res_spin = 0;
 
     // run parameters (dalm_set_params)
     dalm_params prm{};
@@ -329,6 +336,12 @@ int run_sor_on(dalm_ctx* ctx, double* x, const double* b, int slot, double omega
 // (the precision form's hand-over to FP64) instead of starting one
 int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_kind, double pc_omega, int pc_it,
                     long long max_it, double tol, long long* it, double* err, bool resume = false);
+// the same solvers in one launch, for grids that fit a quarter of the compute units
+// (resident.hip): *ran tells whether they applied and finished, with the result in x and
+// in ctx->h_solve
+int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long max_it, double tol, bool* ran);
+int res_bicgstab(dalm_ctx* ctx, double* x, const double* b, int pc_kind, double pc_omega, int pc_it, long long max_it,
+                 double tol, bool* ran);
 int launch_residual(dalm_ctx* ctx, const double* x, const double* b, double* r);
 int launch_Ax(dalm_ctx* ctx, const double* x, double* y);
 int launch_sor_sweep(dalm_ctx* ctx, double* x, const double* b, double omega, int color);

@@ -445,6 +445,10 @@ int dalm_create(dalm_ctx** out, const int64_t size[3], int64_t gc, const double*
         return r;
     };
     if (hipStreamCreate(&ctx->stream) != hipSuccess) return fail(DALM_HIP_ERROR);
+    int device = 0, cus = 0;
+    if (hipGetDevice(&device) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0)
+        ctx->ncu = cus;
     double** one_d[6] = {&ctx->x, &ctx->y, &ctx->z, &ctx->dx, &ctx->dy, &ctx->dz};
     const std::vector<double>* src[6] = {&ctx->hx, &ctx->hy, &ctx->hz, &ctx->hdx, &ctx->hdy, &ctx->hdz};
     for (int q = 0; q < 6; ++q) {
@@ -496,10 +500,10 @@ int dalm_create(dalm_ctx** out, const int64_t size[3], int64_t gc, const double*
         (rc = dev_alloc(ctx, &ctx->counter, 16)) || (rc = dev_alloc(ctx, &ctx->solve, 2)) ||
         (rc = dev_alloc(ctx, &ctx->scal, 1)))
         return fail(rc);
-    if (hipHostMalloc((void**)&ctx->h_solve, 2 * sizeof(SolveState)) != hipSuccess ||
+    if (hipHostMalloc((void**)&ctx->h_solve, 3 * sizeof(SolveState)) != hipSuccess ||
         hipHostMalloc((void**)&ctx->h_scal, sizeof(StepScalars)) != hipSuccess)
         return fail(DALM_HIP_ERROR);
-    std::memset(ctx->h_solve, 0, 2 * sizeof(SolveState));
+    std::memset(ctx->h_solve, 0, 3 * sizeof(SolveState));
     std::memset(ctx->h_scal, 0, sizeof(StepScalars));
     if ((rc = build_operator(ctx))) return fail(rc);
     if (mixed && (rc = setup_mixed(ctx))) return fail(rc);
@@ -547,6 +551,7 @@ int dalm_destroy(dalm_ctx* ctx) {
     for (void* p : ctx->owned_f) (void)hipFree(p);
     if (ctx->alm.box_dev) (void)hipFree(ctx->alm.box_dev);
     if (ctx->counter) (void)hipFree(ctx->counter);
+    if (ctx->res_ring) (void)hipFree(ctx->res_ring);
     if (ctx->solve) (void)hipFree(ctx->solve);
     if (ctx->scal) (void)hipFree(ctx->scal);
     if (ctx->h_solve) (void)hipHostFree(ctx->h_solve);

@@ -762,6 +762,13 @@ int launch_Ax(dalm_ctx* ctx, const double* x, double* y) {
 
 int run_sor_on(dalm_ctx* ctx, double* x, const double* b, int slot, double omega, long long max_it, double tol,
                long long* it, double* err) {
+    bool ran = false;
+    if (int rc = res_sor(ctx, x, b, omega, max_it, tol, &ran)) return rc;
+    if (ran) {
+        *it = ctx->prev_it[slot] = ctx->h_solve->it;
+        *err = ctx->h_solve->err;
+        return ctx->h_solve->status;
+    }
     const double root_n = sqrt((double)ctx->N);
     hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->solve, tol, max_it, root_n);
     LAUNCH_CHECK();
@@ -807,6 +814,13 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
     PCoef A = ctx->coef();
     const Dims& d = ctx->d;
     if (!resume) {
+        bool ran = false;
+        if (int rc = res_bicgstab(ctx, x, b, pc_kind, pc_omega, pc_it, max_it, tol, &ran)) return rc;
+        if (ran) {
+            *it = ctx->prev_it[slot] = ctx->h_solve->it;
+            *err = ctx->h_solve->err;
+            return ctx->h_solve->status;
+        }
         hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->solve, tol, max_it, root_n);
         hipLaunchKernelGGL(k_bi_init, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, A, x, b, ctx->r, ctx->r0,
                            ctx->partials, ctx->counter, ctx->solve);

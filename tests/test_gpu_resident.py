@@ -1,0 +1,122 @@
+"""The one-launch solvers of small grids (csrc/resident.hip) against the oracle: SOR
+iterates bit for bit, BiCGStab's first iterations to the rounding of its dot products
+and its converged solution, over splits into one and several slabs, odd row lengths,
+a last slab of fewer planes, and a stop by the tolerance in mid-solve."""
+import importlib
+
+import numpy as np
+import pytest
+
+from helpers import interior_mask, rand_field, rel_l2, small_mesh
+
+hip = importlib.import_module("3dalm_amd.hip")
+po = importlib.import_module("pyoracle")
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ok():
+    return po.Kernels("oracle")
+
+
+def _problem(ok, shape):
+    mesh = small_mesh(*shape, 1.2)
+    g = po.make_grid(mesh)
+    A = np.zeros((mesh.L, 7))
+    ok.build_A(g, A)
+    p = rand_field(mesh, 71, 1, 0.1)
+    b = rand_field(mesh, 72, 1, 1.0) * interior_mask(mesh)
+    c = hip.Context(mesh)
+    c.upload("p", p)
+    c.upload("b", b)
+    return mesh, g, A, p, b, c
+
+
+# one slab; 64 slabs of one plane; 33 slabs of two planes, the last of one, odd rows;
+# more rows than threads hold at once (several positions per thread); rows longer than
+# two wavefronts
+SHAPES = [(7, 6, 5), (3, 12, 33), (64, 10, 9), (65, 33, 31), (20, 64, 64), (130, 20, 150)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_sor_bits(ok, shape):
+    print(f"[resident sor {shape}]", flush=True)
+    mesh, g, A, p, b, c = _problem(ok, shape)
+    x, r = p.copy(), np.zeros(mesh.L)
+    it, err = po.C.c_int64(), po.C.c_double()
+    run = lambda n, tol: po.lib("oracle")[0].or_run_sor(po.C.byref(g), po.ptr(A), po.ptr(x), po.ptr(b), po.ptr(r), 1.3,
+                                                        po.C.byref(it), n, po.C.byref(err), tol)
+    run(9, 0.0)
+    got = c.run_sor(1.3, 9, 0.0)
+    assert got[0] == it.value == 9 and got[2] == hip.NONCONVERGED
+    assert np.array_equal(c.download("p"), x)
+    # the sum of N squares in another order: N u / 2 relative, and far less in the mean
+    assert abs(got[1] - err.value) <= 1e-13 * err.value
+    # stopped by the tolerance a few iterations on: the iterate of exactly that iteration
+    tol = 0.9 * err.value
+    run(500, tol)
+    got = c.run_sor(1.3, 500, tol)
+    assert got[0] == it.value < 500 and got[2] == hip.OK
+    assert np.array_equal(c.download("p"), x)
+    c.close()
+
+
+@pytest.mark.parametrize("pc", [hip.PC_JACOBI, hip.PC_SOR])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_bicgstab(ok, shape, pc):
+    print(f"[resident bicgstab {shape} pc {pc}]", flush=True)
+    mesh, g, A, p, b, c = _problem(ok, shape)
+    m = interior_mask(mesh)
+    lib = po.lib("oracle")[0]
+    work = np.zeros(9 * mesh.L)
+    it, err = po.C.c_int64(), po.C.c_double()
+    for n, tol in ((2, 0.0), (5000, 1e-13)):
+        x = p.copy()
+        c.upload("p", p)
+        lib.or_run_bicgstab(po.C.byref(g), po.ptr(A), po.ptr(x), po.ptr(b), po.ptr(work), pc, 1.1, 2, po.C.byref(it), n,
+                            po.C.byref(err), tol)
+        git, gerr, st = c.run_bicgstab(pc, 1.1, 2, n, tol)
+        d = rel_l2(c.download("p")[m], x[m])
+        print(f"  {git} against {it.value} iterations, pressure {d:.2e}", flush=True)
+        if n == 2:  # the rounding of the dot products, not yet amplified by the iteration
+            assert git == 2 and st == hip.NONCONVERGED and d <= 1e-13
+            assert abs(gerr - err.value) <= 1e-12 * err.value
+        else:  # both within 1e-13 of the same solution
+            assert st == hip.OK and gerr <= 1e-13 and d <= 1e-10
+        assert np.array_equal(c.download("p")[~m], p[~m])
+    c.close()
+
+
+def test_breakdown_and_nonfinite():
+    """A zero residual is a breakdown before the first iteration; a NaN in b ends the
+    solve after one (as the kernels of larger grids do)."""
+    mesh = small_mesh(12, 9, 10, 1.2)
+    c = hip.Context(mesh)
+    it, err, st = c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, 50, 1e-8)
+    assert (it, err, st) == (0, 0.0, hip.BREAKDOWN)
+    b = np.zeros(mesh.L)
+    b[np.flatnonzero(interior_mask(mesh))[5]] = np.nan
+    c.upload("b", b)
+    it, err, st = c.run_sor(1.2, 50, 1e-8)
+    assert it == 1 and st == hip.NONFINITE
+    c.upload("p", np.zeros(mesh.L))
+    it, err, st = c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, 50, 1e-8)
+    assert it == 1 and st == hip.NONFINITE
+    c.close()
+
+
+def test_falls_back_when_a_wait_ends(ok, monkeypatch):
+    """A block that gives up waiting (a limit of one poll, set by the environment) ends
+    the launch, and the solve runs with one launch per sweep from the same start: the
+    same iterates, then and for the context's later solves."""
+    monkeypatch.setenv("DALM_RESIDENT_SPIN", "1")
+    mesh, g, A, p, b, c = _problem(ok, (40, 20, 24))
+    x, r = p.copy(), np.zeros(mesh.L)
+    it, err = po.C.c_int64(), po.C.c_double()
+    for n in (4, 3):
+        po.lib("oracle")[0].or_run_sor(po.C.byref(g), po.ptr(A), po.ptr(x), po.ptr(b), po.ptr(r), 1.3, po.C.byref(it), n,
+                                       po.C.byref(err), 0.0)
+        got = c.run_sor(1.3, n, 0.0)
+        assert got[0] == n and np.array_equal(c.download("p"), x)
+    c.close()
