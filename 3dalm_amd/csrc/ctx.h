@@ -342,6 +342,7 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
 int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long max_it, double tol, bool* ran);
 int res_bicgstab(dalm_ctx* ctx, double* x, const double* b, int pc_kind, double pc_omega, int pc_it, long long max_it,
                  double tol, bool* ran);
+int res_sor_mixed(dalm_ctx* ctx, double omega, int inner, long long max_it, double tol, bool* ran);
 int launch_residual(dalm_ctx* ctx, const double* x, const double* b, double* r);
 int launch_Ax(dalm_ctx* ctx, const double* x, double* y);
 int launch_sor_sweep(dalm_ctx* ctx, double* x, const double* b, double omega, int color);

@@ -716,6 +716,13 @@ int run_sor_mixed(dalm_ctx* ctx, double omega, long long max_it, double tol, lon
     float* e = ctx->fz;
     ctx->outer_it = 0;
     ctx->fp64_finish_it = 0;
+    bool ran = false;
+    if (int rc = res_sor_mixed(ctx, omega, kSorInner, max_it, tol, &ran)) return rc;
+    if (ran) {
+        *it = ctx->prev_it[0] = ctx->h_solve->it;
+        *err = ctx->h_solve->err;
+        return ctx->h_solve->status;
+    }
     hipLaunchKernelGGL(ks_state_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->solve, tol, max_it,
                        sqrt((double)ctx->N), (double)kSorInner);
     LAUNCH_CHECK();

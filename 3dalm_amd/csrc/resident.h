@@ -18,9 +18,12 @@
 // and carries no data).
 //
 // Four sets of slots alternate.  A set is written again four exchanges later, and by
-// then its reader's kEmpty has landed: a thread waits for its stores (xchg_fence) before
-// the barrier that precedes its block's next publication, and the writer has seen that
-// publication.  All slots are empty when a launch ends.
+// then its reader's kEmpty has landed: a thread waits for its earlier stores (xchg_fence)
+// when it has taken its words, before it empties them.  So the kEmpty of exchange n has
+// landed before the barrier that ends exchange n + 1, which precedes the block's
+// publication n + 2, and the writer has seen publication n + 3 when it writes again.
+// (Waiting for them at once, ahead of the barrier, cost a store's way to memory in every
+// exchange.)  All slots are empty when a launch ends.
 //
 // Progress.  The blocks wait for each other, so all of them must be on the GPU at
 // once: one block fits a compute unit, and no launch has more than a quarter of the
@@ -177,8 +180,10 @@ struct ResSync {
 // phase's marks go to the other one.  Returns false when the block is to leave.
 template <int M>
 __device__ __forceinline__ bool res_barrier(ResSync& sh, ResThread<M>& t) {
-    xchg_fence();
-    __syncthreads();
+    // LDS only: the exchange's stores are not waited for here
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     const bool ok = sh.bad[t.phase & 1] == 0;
     ++t.phase;
     return ok;
@@ -245,6 +250,7 @@ __device__ __forceinline__ void res_take(const Dims& d, const ResShape& s, ResTh
                 if (a[m] == S::empty) a[m] = slot_load(lo + j * s.nk + t.k);
                 if (b[m] == S::empty) b[m] = slot_load(hi + j * s.nk + t.k);
             }
+            if (m == 0) xchg_fence();  // the stores of this exchange's publication and before
             const int at = (j + 1) * s.pk + t.k + 1;
             if (nl[m]) {
                 slot_store(lo + j * s.nk + t.k, S::empty);
@@ -305,6 +311,7 @@ __device__ __forceinline__ void res_sum_take(const ResShape& s, ResThread<M>& t,
                 }
                 w[q] = slot_load(set + (size_t)q * s.blocks + lane);
             }
+            if (q == 0) xchg_fence();
             if (lane < s.blocks) slot_store(set + (size_t)q * s.blocks + lane, kEmpty);
             const double v = wave_total(SlotWord<double>::value(w[q]));
             if (lane == 0) sh.out[q] = v;
@@ -329,7 +336,8 @@ __device__ __forceinline__ bool res_sum(const double (&v)[NV], const ResShape& s
 ResShape res_shape(const dalm_ctx* ctx, int lanes, size_t bytes);
 // allocate and empty the exchange slots on first use (sets ctx->res_off without room)
 int res_prepare(dalm_ctx* ctx, ResShape& s);
-// wait for the launch and read its SolveState; *aborted when its result is to be dropped
-int res_finish(dalm_ctx* ctx, bool* aborted);
-// interior of x <- interior of from
-int res_commit(dalm_ctx* ctx, double* x, const double* from);
+// whether this context may run a resident solve of up to max_it iterations now
+bool res_may_run(const dalm_ctx* ctx, long long max_it);
+// wait for the launch, read its SolveState and copy its result, in ctx->r, to the
+// interior of x; *ran is false when the launch was aborted (x is then as it was)
+int res_finish(dalm_ctx* ctx, double* x, bool* ran);

@@ -5,10 +5,10 @@
 // What bounds them is the chain of dependent phases of an iteration (a colour sweep, a
 // Jacobi sweep, a product, a sum over the grid), each a store that must reach the
 // neighbour and be read: 1.2 to 1.5 us against the 4.7 us of a launch.  The work inside
-// a phase is 0.1 to 0.5 us.  Per iteration, in microseconds, one launch per sweep and
-// resident: SOR 64x32x32 15.3 and 3.3, 64x48x48 17.5 and 5.6; BiCGStab with three Jacobi
-// sweeps 20x12x12 37.7 and 14.1, 64x32x32 42.8 and 18.5, with two SOR sweeps 52.6 and 17.5,
-// 60.2 and 22.8.
+// a phase is 0.1 to 0.8 us.  Per iteration, in microseconds, one launch per sweep and
+// resident: SOR 64x32x32 15.3 and 3.0, 64x48x48 17.5 and 5.2; BiCGStab with three Jacobi
+// sweeps 20x12x12 37.7 and 12.5, 64x32x32 42.8 and 16.5, with two SOR sweeps 52.6 and 15.5,
+// 60.2 and 20.5.
 //
 // Per cell the arithmetic is that of the one-launch-per-sweep kernels in poisson.hip
 // (the same operands in the same order, division included), so SOR iterates are the
@@ -411,8 +411,9 @@ int res_prepare(dalm_ctx* ctx, ResShape& s) {
     // slots for the largest split of this grid: one word per cell of a plane, direction,
     // block and set
     const Dims& d = ctx->d;
-    const size_t ring = (size_t)kSlotSets * 2 * kResMaxBlocks * d.ny * d.nz;
-    const size_t gath = (size_t)kSlotSets * kResMaxBlocks * 4 * kResMaxBlocks;
+    const size_t most = d.nx < kResMaxBlocks ? d.nx : kResMaxBlocks;
+    const size_t ring = (size_t)kSlotSets * 2 * most * d.ny * d.nz;
+    const size_t gath = (size_t)kSlotSets * most * 4 * most;
     if (!ctx->res_ring) {
         if (hipMalloc(&ctx->res_ring, (ring + gath) * sizeof(u64w) + ring * sizeof(unsigned) + 64) != hipSuccess) {
             (void)hipGetLastError();  // no room for the slots: the launches per sweep need none
@@ -439,30 +440,32 @@ int res_prepare(dalm_ctx* ctx, ResShape& s) {
     return DALM_OK;
 }
 
-int res_finish(dalm_ctx* ctx, bool* aborted) {
+int res_finish(dalm_ctx* ctx, double* x, bool* ran) {
     int* flag = (int*)(ctx->h_solve + 2);
     HIP_TRY(hipMemcpyAsync(ctx->h_solve, ctx->solve, sizeof(SolveState), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipMemcpyAsync(flag, ctx->res_abort, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    *aborted = *flag != 0;
-    // something keeps this context's blocks off the GPU: it does not wait for that again
-    if (*aborted) ctx->res_off = true;
-    return DALM_OK;
-}
-
-int res_commit(dalm_ctx* ctx, double* x, const double* from) {
-    hipLaunchKernelGGL(k_res_commit, dim3(ctx->grid), dim3(BLOCK), 0, ctx->stream, ctx->d, x, from);
+    if (*flag != 0) {
+        // something keeps this context's blocks off the GPU: it does not wait for that again
+        ctx->res_off = true;
+        return DALM_OK;
+    }
+    hipLaunchKernelGGL(k_res_commit, dim3(ctx->grid), dim3(BLOCK), 0, ctx->stream, ctx->d, x, (const double*)ctx->r);
     HIP_TRY(hipGetLastError());
+    *ran = true;
     return DALM_OK;
 }
 
 // A solve that may run longer than this keeps the launches per sweep (the GPU stays
-// available to other programs between them).
+// available to other programs between them), and so does one whose launches are timed.
 constexpr long long kResMaxIterations = 20000;
+bool res_may_run(const dalm_ctx* ctx, long long max_it) {
+    return !ctx->res_off && max_it <= kResMaxIterations && ctx->probe.kernel == 0;
+}
 
 int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long max_it, double tol, bool* ran) {
     *ran = false;
-    if (ctx->res_off || max_it > kResMaxIterations || ctx->probe.kernel != 0) return DALM_OK;
+    if (!res_may_run(ctx, max_it)) return DALM_OK;
     ResShape s = res_shape(ctx, (ctx->d.nz + 1) / 2, 2 * sizeof(double));
     if (s.blocks == 0) return DALM_OK;
     if (int rc = res_prepare(ctx, s)) return rc;
@@ -479,18 +482,13 @@ int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long m
     default: launch(k_res_sor<4>); break;
     }
     HIP_TRY(hipGetLastError());
-    bool aborted = false;
-    if (int rc = res_finish(ctx, &aborted)) return rc;
-    if (aborted) return DALM_OK;
-    if (int rc = res_commit(ctx, x, ctx->r)) return rc;
-    *ran = true;
-    return DALM_OK;
+    return res_finish(ctx, x, ran);
 }
 
 int res_bicgstab(dalm_ctx* ctx, double* x, const double* b, int pc_kind, double pc_omega, int pc_it, long long max_it,
                  double tol, bool* ran) {
     *ran = false;
-    if (ctx->res_off || max_it > kResMaxIterations || pc_it < 1 || ctx->probe.kernel != 0) return DALM_OK;
+    if (!res_may_run(ctx, max_it) || pc_it < 1) return DALM_OK;
     ResShape s = res_shape(ctx, ctx->d.nz, sizeof(double));
     if (s.blocks == 0) return DALM_OK;
     if (int rc = res_prepare(ctx, s)) return rc;
@@ -508,10 +506,5 @@ int res_bicgstab(dalm_ctx* ctx, double* x, const double* b, int pc_kind, double 
     default: jac ? launch(k_res_bicgstab<4, true>) : launch(k_res_bicgstab<4, false>); break;
     }
     HIP_TRY(hipGetLastError());
-    bool aborted = false;
-    if (int rc = res_finish(ctx, &aborted)) return rc;
-    if (aborted) return DALM_OK;
-    if (int rc = res_commit(ctx, x, ctx->r)) return rc;
-    *ran = true;
-    return DALM_OK;
+    return res_finish(ctx, x, ran);
 }

@@ -120,3 +120,30 @@ def test_falls_back_when_a_wait_ends(ok, monkeypatch):
         got = c.run_sor(1.3, n, 0.0)
         assert got[0] == n and np.array_equal(c.download("p"), x)
     c.close()
+
+
+@pytest.mark.parametrize("shape", [(7, 6, 5), (64, 10, 9), (65, 33, 31), (20, 64, 64)])
+def test_sor_mixed(shape):
+    """The precision form's SOR of one step against the FP64 oracle's: after the same
+    number of iterations (a multiple of 8) the pressure and the residual differ by the
+    FP32 rounding of the corrections, 2^-24 of each (allowed: ten of them), and by that of
+    the FP32 predictor in b."""
+    cases, solver = importlib.import_module("3dalm_amd.cases"), importlib.import_module("3dalm_amd.solver")
+    print(f"[resident sor mixed {shape}]", flush=True)
+    case = cases.case_c1(*shape, steps=1)
+    case.max_it, case.tol = 24, 0.0
+    o, s = po.OracleSolver(case), solver.Solver(case, hip.MIXED)
+    try:
+        so, sm = o.step(), s.step()
+        assert sm["it"] == so["it"] == 24
+        m = interior_mask(case.mesh)
+        d = rel_l2(s.field("p")[m], o.field("p")[m])
+        print(f"  pressure {d:.2e}, err {sm['err']:.6e} against {so['err']:.6e}", flush=True)
+        assert d <= 10 * 2.0 ** -24 * 10 and abs(sm["err"] - so["err"]) <= 1e-5 * so["err"]
+        case.max_it, case.tol = 2000, 0.5 * so["err"]
+        s2 = solver.Solver(case, hip.MIXED)
+        st = s2.step()
+        assert st["it"] % 8 == 0 and st["it"] < 2000 and st["err"] <= case.tol
+        s2.close()
+    finally:
+        s.close()
