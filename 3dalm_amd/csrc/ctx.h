@@ -180,6 +180,18 @@ struct AdjointState {
     double replay_ms = 0, reverse_ms = 0;
 };
 
+// The split of the precision form's fused half-iterations (fused_mixed.hip): a block's R
+// rows x Q quads of four cells, the j and k tiles, planes per unit; `mode` selects the
+// kernel (0 any row length, 1 a multiple of four, 2 rows of 256, whose iteration leaves
+// r and x to later kernels).
+struct HalfGeom {
+    int R, Q, tj, tk, ni;
+    int blocks, threads, mode;
+    int sums;   // partial sums of each dot product
+    bool cols;  // they are those of the separate kernels' units, in the same order
+    size_t lds;
+};
+
 struct dalm_ctx {
     Dims d;
     long long L = 0, N = 0;
@@ -229,6 +241,8 @@ struct dalm_ctx {
     // kXGroupF, so that an outstanding pressure update keeps its z), allocated on first use
     float* fzx[kXGroupF - 1] = {};
     float* fz2x[kXGroupF - 1] = {};
+    HalfGeom half{};
+    bool have_half = false;
     MetricF mf{};
     PCoefF pcf{};
     std::vector<void*> owned_f;   // float 1-D arrays behind mf / pcf
@@ -360,15 +374,16 @@ int ensure_adjoint_buffers(dalm_ctx* ctx);
 int sync_stream(dalm_ctx* ctx);
 int zero_device(dalm_ctx* ctx, double* a, long long n);
 // fused half-iterations of the precision form's BiCGStab (fused_mixed.hip)
-bool fused_half_applies(const dalm_ctx* ctx, int pc_kind, int pc_it);
-int fused_half_grid(const dalm_ctx* ctx, int* ni);
+// their split of this grid, or null where the fused path does not apply
+const HalfGeom* half_geom(dalm_ctx* ctx, int pc_kind, int pc_it);
 // planes per unit of a fused kernel that runs one block per compute unit over
 // `tiles` j tiles: as many plane chunks as fill the compute units once, chunks of at
 // least 16 planes
 int fused_planes(const dalm_ctx* ctx, int tiles);
 // the fused half-iterations: z_p into zp_out, z_s into zs_out
-int launch_half_p(dalm_ctx* ctx, const float* p_in, const float* q_in, float* p_out, float* q_out, float* zp_out);
-int launch_half_s(dalm_ctx* ctx, const float* q, float* zs_out);
+int launch_half_p(dalm_ctx* ctx, const HalfGeom& G, const float* p_in, const float* q_in, float* p_out, float* q_out,
+                  float* zp_out);
+int launch_half_s(dalm_ctx* ctx, const HalfGeom& G, const float* q, float* zs_out);
 
 // the pressure update of a precision-form iteration, x + alpha z_p + omega z_s, in one
 // expression wherever it is evaluated (the fused p-half, the replacement and the flush)

@@ -773,12 +773,18 @@ int run_poisson_mixed(dalm_ctx* ctx, int pc_kind, double pc_omega, int pc_it, lo
     // rows of a multiple of 256 interior cells: the four-per-lane Jacobi sweep
     const bool vec4 = vec4_applies(d);
     const int grid4 = d.tj * vec4_tiles(d) * d.nch;
-    // rows of exactly 256 cells with three Jacobi sweeps: each half-iteration is one
-    // fused kernel (fused_mixed.hip); p and q alternate between a buffer pair (the
-    // Jacobi partners, which the fused path does not use)
-    const bool fused = fused_half_applies(ctx, pc_kind, pc_it);
-    int fni = 0;
-    const int fgrid = fused ? fused_half_grid(ctx, &fni) : 0;
+    // three Jacobi sweeps: each half-iteration is one fused kernel (fused_mixed.hip); p and
+    // q alternate between a buffer pair (the Jacobi partners, which the fused path does
+    // not use)
+    const HalfGeom* split = half_geom(ctx, pc_kind, pc_it);
+    const bool halves = split != nullptr;
+    const HalfGeom fgeom = halves ? *split : HalfGeom{};
+    const int fgrid = fgeom.sums;
+    // rows of 256 cells: the p-half also forms r, and x follows every kXGroupF iterations.
+    // Other rows keep kg_xr after the s-half, so that <r0, r> is that of the stored r, as in
+    // the separate kernels: the iterates are theirs (<r0, s> - omega <r0, t> differs from it
+    // by r's rounding, and BiCGStab doubles such a difference every iteration).
+    const bool fused = halves && fgeom.mode == 2;
     if (fused) {
         if (const int rz = ensure_fused_z(ctx)) return rz;
     }
@@ -911,13 +917,13 @@ int run_poisson_mixed(dalm_ctx* ctx, int pc_kind, double pc_omega, int pc_it, lo
                     float* P[2] = {ctx->fp, ctx->ftmp};
                     float* Q[2] = {ctx->fq, ctx->ftmp2};
                     probe_begin(ctx, DALM_K_HALF_P_MIXED);
-                    if ((rc = launch_half_p(ctx, P[k & 1], Q[k & 1], P[(k + 1) & 1], Q[(k + 1) & 1],
+                    if ((rc = launch_half_p(ctx, fgeom, P[k & 1], Q[k & 1], P[(k + 1) & 1], Q[(k + 1) & 1],
                                             ZP[k % kXGroupF])))
                         return dalm_fail_msg(ctx, rc, "fused p half-iteration launch");
                     probe_end(ctx, DALM_K_HALF_P_MIXED);
                     if ((rc = launch_finalize(ctx, FIN_ALPHA, fgrid, st, nullptr))) return rc;
                     probe_begin(ctx, DALM_K_HALF_S_MIXED);
-                    if ((rc = launch_half_s(ctx, Q[(k + 1) & 1], ZS[k % kXGroupF])))
+                    if ((rc = launch_half_s(ctx, fgeom, Q[(k + 1) & 1], ZS[k % kXGroupF])))
                         return dalm_fail_msg(ctx, rc, "fused s half-iteration launch");
                     probe_end(ctx, DALM_K_HALF_S_MIXED);
                     if ((rc = launch_finalize(ctx, FIN_MX_OMEGA, fgrid, st, nullptr))) return rc;
@@ -928,42 +934,60 @@ int run_poisson_mixed(dalm_ctx* ctx, int pc_kind, double pc_omega, int pc_it, lo
                     if ((rc = launch_finalize(ctx, FIN_MX_RU, ctx->sgrid, st, nullptr))) return rc;
                     continue;
                 }
-                probe_begin(ctx, DALM_K_PUPDATE_MIXED);
-                if (vec4)
-                    hipLaunchKernelGGL(kg_p4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fp,
-                                       ctx->fq, ctx->fz, pc_first, (const SolveState*)st);
-                else
-                    hipLaunchKernelGGL(kg_p, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fp,
-                                       ctx->fq, ctx->fz, pc_first, (const SolveState*)st);
-                probe_end(ctx, DALM_K_PUPDATE_MIXED);
-                float* zp = precondition(ctx->fz, ctx->ftmp, ctx->fp);
-                probe_begin(ctx, DALM_K_SPMV_MIXED);
-                if (vec4)
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv4<0>), dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A,
-                                       zp, ctx->fq, ctx->fr0, ctx->partials, (const SolveState*)st);
-                else
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv<0>), dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d,
-                                       A, zp, ctx->fq, ctx->fr0, ctx->partials, (const SolveState*)st);
-                probe_end(ctx, DALM_K_SPMV_MIXED);
-                if ((rc = launch_finalize(ctx, FIN_ALPHA, vec4 ? grid4 : ctx->sgrid, st, nullptr))) return rc;
-                probe_begin(ctx, DALM_K_SUPDATE_MIXED);
-                if (vec4)
-                    hipLaunchKernelGGL(kg_s4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fq,
-                                       ctx->fs, ctx->fz2, pc_first, (const SolveState*)st);
-                else
-                    hipLaunchKernelGGL(kg_s, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fq,
-                                       ctx->fs, ctx->fz2, pc_first, (const SolveState*)st);
-                probe_end(ctx, DALM_K_SUPDATE_MIXED);
-                float* zs = precondition(ctx->fz2, ctx->ftmp2, ctx->fs);
-                probe_begin(ctx, DALM_K_SPMV_MIXED);
-                if (vec4)
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv4<1>), dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A,
-                                       zs, ctx->ft, ctx->fs, ctx->partials, (const SolveState*)st);
-                else
-                    hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv<1>), dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d,
-                                       A, zs, ctx->ft, ctx->fs, ctx->partials, (const SolveState*)st);
-                probe_end(ctx, DALM_K_SPMV_MIXED);
-                if ((rc = launch_finalize(ctx, FIN_OMEGA, vec4 ? grid4 : ctx->sgrid, st, nullptr))) return rc;
+                float *zp = ctx->fz, *zs = ctx->fz2;
+                const long long k = launched + c;
+                float *const P[2] = {ctx->fp, ctx->ftmp}, *const Q[2] = {ctx->fq, ctx->ftmp2};
+                if (halves) {
+                    probe_begin(ctx, DALM_K_HALF_P_MIXED);
+                    if ((rc = launch_half_p(ctx, fgeom, P[k & 1], Q[k & 1], P[(k + 1) & 1], Q[(k + 1) & 1], zp)))
+                        return dalm_fail_msg(ctx, rc, "fused p half-iteration launch");
+                    probe_end(ctx, DALM_K_HALF_P_MIXED);
+                } else {
+                    probe_begin(ctx, DALM_K_PUPDATE_MIXED);
+                    if (vec4)
+                        hipLaunchKernelGGL(kg_p4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fp,
+                                           ctx->fq, ctx->fz, pc_first, (const SolveState*)st);
+                    else
+                        hipLaunchKernelGGL(kg_p, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fp,
+                                           ctx->fq, ctx->fz, pc_first, (const SolveState*)st);
+                    probe_end(ctx, DALM_K_PUPDATE_MIXED);
+                    zp = precondition(ctx->fz, ctx->ftmp, ctx->fp);
+                    probe_begin(ctx, DALM_K_SPMV_MIXED);
+                    if (vec4)
+                        hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv4<0>), dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A,
+                                           zp, ctx->fq, ctx->fr0, ctx->partials, (const SolveState*)st);
+                    else
+                        hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv<0>), dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d,
+                                           A, zp, ctx->fq, ctx->fr0, ctx->partials, (const SolveState*)st);
+                    probe_end(ctx, DALM_K_SPMV_MIXED);
+                }
+                const int dots = halves ? fgrid : vec4 ? grid4 : ctx->sgrid;
+                if ((rc = launch_finalize(ctx, FIN_ALPHA, dots, st, nullptr))) return rc;
+                if (halves) {
+                    probe_begin(ctx, DALM_K_HALF_S_MIXED);
+                    if ((rc = launch_half_s(ctx, fgeom, Q[(k + 1) & 1], zs)))
+                        return dalm_fail_msg(ctx, rc, "fused s half-iteration launch");
+                    probe_end(ctx, DALM_K_HALF_S_MIXED);
+                } else {
+                    probe_begin(ctx, DALM_K_SUPDATE_MIXED);
+                    if (vec4)
+                        hipLaunchKernelGGL(kg_s4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fq,
+                                           ctx->fs, ctx->fz2, pc_first, (const SolveState*)st);
+                    else
+                        hipLaunchKernelGGL(kg_s, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, Af, ctx->fr, ctx->fq,
+                                           ctx->fs, ctx->fz2, pc_first, (const SolveState*)st);
+                    probe_end(ctx, DALM_K_SUPDATE_MIXED);
+                    zs = precondition(ctx->fz2, ctx->ftmp2, ctx->fs);
+                    probe_begin(ctx, DALM_K_SPMV_MIXED);
+                    if (vec4)
+                        hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv4<1>), dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A,
+                                           zs, ctx->ft, ctx->fs, ctx->partials, (const SolveState*)st);
+                    else
+                        hipLaunchKernelGGL(HIP_KERNEL_NAME(kg_spmv<1>), dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d,
+                                           A, zs, ctx->ft, ctx->fs, ctx->partials, (const SolveState*)st);
+                    probe_end(ctx, DALM_K_SPMV_MIXED);
+                }
+                if ((rc = launch_finalize(ctx, FIN_OMEGA, dots, st, nullptr))) return rc;
                 probe_begin(ctx, DALM_K_UPDATE_MIXED);
                 if (vec4)
                     hipLaunchKernelGGL(kg_xr4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, ctx->p, zp, zs, ctx->fs,
@@ -1013,7 +1037,7 @@ int run_poisson_mixed(dalm_ctx* ctx, int pc_kind, double pc_omega, int pc_it, lo
             flush(h, ctx->p);
             LAUNCH_CHECK();
         }
-        if (fused && (h.it & 1)) {
+        if (halves && (h.it & 1)) {
             // after an odd number of iterations the current p and q are the partners
             std::swap(ctx->fp, ctx->ftmp);
             std::swap(ctx->fq, ctx->ftmp2);

@@ -23,6 +23,11 @@ struct FinArgs {
 };
 
 __global__ __launch_bounds__(BLOCK) void k_finalize(FinArgs a) {
+    // no residual replacement was due (most iterations): nothing to sum
+    if (a.mode == FIN_MX_RU && !a.st->ru) {
+        if (threadIdx.x == 0 && !a.st->done && a.st->xdef >= kXGroupF) a.st->xdef = 0;  // as below
+        return;
+    }
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if (a.mode == FIN_MX_OMEGA) {
         reduce_partials<5>(a.partials, a.nb, s);

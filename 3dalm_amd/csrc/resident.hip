@@ -57,7 +57,7 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_sor(Dims d, PCoef A, Res
                                                          const double* __restrict__ b, double* __restrict__ out,
                                                          double omega, long long max_it, double tol, double root_n,
                                                          SolveState* st) {
-    extern __shared__ double slab[];
+    extern __shared__ __align__(16) double slab[];
     __shared__ ResSync sh;
     if (threadIdx.x < 2) sh.bad[threadIdx.x] = 0;
     ResThread<M> t = res_thread<M>(d, s);
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_bicgstab(Dims d, PCoef A
                                                               const double* __restrict__ b, double* __restrict__ out,
                                                               double pc_omega, int pc_it, long long max_it, double tol,
                                                               double root_n, SolveState* st) {
-    extern __shared__ double slab[];
+    extern __shared__ __align__(16) double slab[];
     __shared__ ResSync sh;
     if (threadIdx.x < 2) sh.bad[threadIdx.x] = 0;
     ResThread<M> t = res_thread<M>(d, s);

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_sor_mixed(Dims d, PCoef 
                                                                   double* __restrict__ out, float omega, int inner,
                                                                   long long max_it, double tol, double root_n,
                                                                   SolveState* st) {
-    extern __shared__ double slab[];  // the residual's x, then the sweeps' e (as floats)
+    extern __shared__ __align__(16) double slab[];  // the residual's x, then the sweeps' e (as floats)
     float* const eslab = (float*)slab;
     __shared__ ResSync sh;
     if (threadIdx.x < 2) sh.bad[threadIdx.x] = 0;

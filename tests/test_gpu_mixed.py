@@ -158,3 +158,31 @@ def test_mixed_passes_and_fp64_hand_over(builder, cap):
         assert rel_l2(s.field("U")[m], o.field("U")[m]) <= 1e-4
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("interior, iters", [(s, n) for s in ((9, 10, 13), (33, 30, 87), (40, 24, 64), (70, 13, 30),
+                                                              (82, 20, 643), (12, 10, 256)) for n in (1, 2, 9)] +
+                         [((131, 130, 125), 2), ((129, 127, 132), 2), ((50, 150, 283), 2)])
+def test_fused_half_iterations(interior, iters):
+    """The fused half-iterations on rows of any length (quads that reach beyond the row,
+    rows cut into k tiles, a last j tile and a last plane chunk of fewer cells, rows of 256
+    cells; from two million cells on chunks and tiles of whole units): the pressure after the first iterations of a step against the FP64
+    oracle's.  An iteration rounds each vector about 16 times to FP32 (2^-24), and
+    BiCGStab lets that grow by up to a factor 3 per iteration; a cell, row or update left
+    out is off by more than 1e-3.  After 9 iterations one group of eight pressure updates
+    has been applied and one is outstanding."""
+    case = cases.case_c1(*interior, steps=1)
+    case.method, case.pc, case.pc_it, case.max_it, case.tol = "BiCG", "Jacobi", 3, iters, 0.0
+    print(f"[fused halves {interior} {iters} iterations]", flush=True)
+    o, s = po.OracleSolver(case), solver.Solver(case, hip.MIXED)
+    try:
+        so, sm = o.step(), s.step()
+        assert sm["it"] == so["it"] == iters
+        m = interior_mask(case.mesh)
+        d = rel_l2(s.field("p")[m], o.field("p")[m])
+        print(f"  pressure {d:.2e}", flush=True)
+        assert d <= 16 * 2.0 ** -24 * 3.0 ** (iters - 1) * 4
+        outside = s.field("p")[~m]
+        assert np.all(np.isfinite(outside))
+    finally:
+        s.close()
