@@ -258,6 +258,9 @@ struct dalm_ctx {
     unsigned* counter = nullptr;
     SolveState* solve = nullptr;   // device
     SolveState* h_solve = nullptr; // pinned host mirror
+    double* out_pin = nullptr;     // two pinned slots of copy_out (at most 16 MiB), on first use
+    long long out_slot = 0;
+    hipEvent_t out_ev[2] = {};
     StepScalars* scal = nullptr;   // device
     StepScalars* h_scal = nullptr; // pinned host
 
@@ -372,6 +375,8 @@ int adjoint_record_from(dalm_ctx* src, int status);
 void adjoint_free(dalm_ctx* ctx);
 int ensure_adjoint_buffers(dalm_ctx* ctx);
 int sync_stream(dalm_ctx* ctx);
+// device components c[0..nc) to host as host[cell * nc + q] (copyout.hip)
+int copy_out(dalm_ctx* ctx, void* const c[3], int nc, bool f32, double* host);
 int zero_device(dalm_ctx* ctx, double* a, long long n);
 // fused half-iterations of the precision form's BiCGStab (fused_mixed.hip)
 // their split of this grid, or null where the fused path does not apply

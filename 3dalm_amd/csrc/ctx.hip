@@ -556,6 +556,9 @@ int dalm_destroy(dalm_ctx* ctx) {
     if (ctx->scal) (void)hipFree(ctx->scal);
     if (ctx->h_solve) (void)hipHostFree(ctx->h_solve);
     if (ctx->h_scal) (void)hipHostFree(ctx->h_scal);
+    if (ctx->out_pin) (void)hipHostFree(ctx->out_pin);
+    for (hipEvent_t e : ctx->out_ev)
+        if (e) (void)hipEventDestroy(e);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return DALM_OK;
@@ -599,18 +602,7 @@ int dalm_download(dalm_ctx* ctx, int64_t field, double* host) {
     bool f32;
     TRY(field_ptrs(ctx, field, c, &nc, &f32));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    std::vector<double> tmp(f32 ? 0 : ctx->L);
-    std::vector<float> tmpf(f32 ? ctx->L : 0);
-    for (int q = 0; q < nc; ++q) {
-        if (f32) {
-            HIP_TRY(hipMemcpy(tmpf.data(), c[q], ctx->L * sizeof(float), hipMemcpyDeviceToHost));
-            for (long long e = 0; e < ctx->L; ++e) host[e * nc + q] = tmpf[e];
-        } else {
-            HIP_TRY(hipMemcpy(tmp.data(), c[q], ctx->L * sizeof(double), hipMemcpyDeviceToHost));
-            for (long long e = 0; e < ctx->L; ++e) host[e * nc + q] = tmp[e];
-        }
-    }
-    return DALM_OK;
+    return copy_out(ctx, c, nc, f32, host);
 }
 
 int dalm_set_params(dalm_ctx* ctx, const dalm_params* prm) {
