@@ -562,6 +562,7 @@ constexpr int kFRows = 12;
 constexpr int kFOwn = kFRows - 4;
 constexpr int kFLag = 2;
 constexpr int kFPad = 4;
+constexpr int kPcThreads = 64 * kFRows;
 constexpr int kFRowLen = 256 + 2 * kFPad;
 typedef double d4a __attribute__((ext_vector_type(kVecK), aligned(32)));
 
@@ -703,6 +704,194 @@ __global__ __launch_bounds__(64 * kFRows) void k_half_pc4(Dims d, PCoef A, const
     }
 }
 
+// k_half_pc4 on rows of other lengths: a block of R rows x Q quads (one thread per quad)
+// with rows as long as they are, so that a wavefront may hold parts of several rows.
+// Nothing outside the grid is masked but the loads' values: off-diagonals of ghost planes,
+// rows and cells are zero, so the sweeps leave those cells zero (their diagonals are not: a
+// ghost cell along k gets one), and a quad's cells beyond its row are cleared when it is
+// loaded and stored.  The same arithmetic per cell, so the same bits as the update and the
+// sweeps one by one, which move 11 + 10 vectors an iteration through memory against 5 + 4.
+// Bound by memory on large grids, by the steps' issue (FP64 divisions, LDS) on small ones.  A
+// step of 10 to 16 iterations before and with it: 973 and 959 us at 70x60x60, 2994 and 2738 at
+// 192x96x96, 5087 and 4244 at 256x128x128, 7225 and 5815 at 300x150x150, 14885 and 10243 at
+// 400x200x190, 24050 and 17125 at 480x180x290.  A row's plane lies in LDS as the quads' first pairs of cells and then
+// their second ones, so that a wavefront's 16-byte reads are consecutive.
+template <int WHICH>
+__global__ __launch_bounds__(kPcThreads) void k_half_pc(Dims d, PCoef A, const double* __restrict__ r,
+                                                       const double* __restrict__ vin, const double* __restrict__ q,
+                                                       double* __restrict__ vout, double* __restrict__ zout,
+                                                       HalfGeom G, const SolveState* st) {
+    if (st->done) return;
+    extern __shared__ __align__(16) double pc_sh[];
+    const int Q = G.Q, half = 2 * (Q + 2), len = 2 * half, plane = G.R * len, nk = 4 * Q;
+    double *const at = pc_sh, *const ab = at + nk, *const atu = ab + nk, *const abu = atu + nk;
+    double* const lv = abu + nk;  // [2 copies][2 levels][R][len]
+    const int row = (int)threadIdx.x / Q, lane = (int)threadIdx.x % Q;
+    const int g = d.gc;
+    // j tile fastest, a contiguous range of units per XCD (as kg_half4)
+    const int u = xcd_unit((int)blockIdx.x, (int)gridDim.x);
+    const int jt = u % G.tj, ic = u / G.tj, ni = G.ni;
+    const int own0 = g + ic * ni;
+    int i1 = own0 + ni;
+    if (i1 > g + d.nx) i1 = g + d.nx;
+    const int i0 = i1 - ni;
+    const int j = g + jt * (G.R - 2 * kFLag) + row - kFLag;
+    const bool jin = row < G.R && j >= g && j < g + d.ny;
+    const bool owned = jin && row >= kFLag && row < G.R - kFLag;
+    const int jc = j < 0 ? 0 : (j < d.n1 ? j : d.n1 - 1), left = d.nz - 4 * lane;
+    const int at_jk = jc * d.sj + g + 4 * lane;
+    const double beta = st->beta, om = st->omega, alpha = st->alpha;
+    const bool first = st->it == 0;
+    const double an = A.an[jc], as = A.as[jc], anu = A.anu[jc], asu = A.asu[jc];
+    for (int t = threadIdx.x; t < nk; t += blockDim.x) {
+        const int k = g + t, td = (t & 3) * Q + (t >> 2);
+        const bool in = t < d.nz;
+        at[td] = in ? A.at[k] : 0.0;
+        ab[td] = in ? A.ab[k] : 0.0;
+        atu[td] = in ? A.atu[k] : 1.0;
+        abu[td] = in ? A.abu[k] : 0.0;
+    }
+    for (int t = threadIdx.x; t < 4 * plane; t += blockDim.x) lv[t] = 0.0;
+    __syncthreads();
+
+    typedef double d2a __attribute__((ext_vector_type(2), aligned(16)));
+    const d4k zero = {0.0, 0.0, 0.0, 0.0};
+    d4k z1a = zero, z1b = zero, z2a = zero, z2b = zero, va = zero, vb = zero;
+    const auto inner = [&](int i) { return i >= g && i < g + d.nx; };
+    const auto clamp_i = [&](int i) { return i < 0 ? 0 : (i < d.n0 ? i : d.n0 - 1); };
+    const auto at_plane = [&](const double* p, int i) {
+        d4k x = ld4(p, clamp_i(i) * d.si + at_jk);
+        const bool ok = jin && inner(i);
+#pragma unroll
+        for (int m = 0; m < kVecK; ++m) x[m] = ok && m < left ? x[m] : 0.0;
+        return x;
+    };
+    const auto put = [&](double* p, int i, d4k x) {
+#pragma unroll
+        for (int m = 0; m < kVecK; ++m) x[m] = m < left ? x[m] : 0.0;
+        __builtin_nontemporal_store(x, (d4k*)(p + i * d.si + at_jk));
+    };
+    struct In {
+        d4k r, v, q;
+    };
+    const auto load0 = [&](int i) {
+        In x;
+        x.r = at_plane(r, i);
+        x.q = at_plane(q, i);
+        if (WHICH == 0) x.v = at_plane(vin, i);
+        return x;
+    };
+    const int rr = row == 0 ? 1 : (row >= G.R - 1 ? G.R - 2 : row);  // neighbour rows stay in range
+    const int me = row * len + 2 * (lane + 1), near = rr * len + 2 * (lane + 1);
+    struct Nb {
+        d4k n, s;
+        double kb, kf;
+    };
+    const auto quad = [&](const double* p) {
+        const d2a a = *(const d2a*)p, b = *(const d2a*)(p + half);
+        return d4k{a[0], a[1], b[0], b[1]};
+    };
+    const auto nbrs = [&](const double* p) {
+        Nb b;
+        b.n = quad(p + len);
+        b.s = quad(p - len);
+        b.kb = p[half - 1];
+        b.kf = p[2];
+        return b;
+    };
+    constexpr bool carry = WHICH == 1;  // as in k_half_pc4
+    const auto sweep = [&](int i, const Nb& nb, const d4k& xb, const d4k& xa, const d4k& xn, const d4k& rhs,
+                           const d4k& acv) {
+        const int ip = clamp_i(i);
+        const double acj = (A.acx[ip] - anu) - asu, ae = A.ae[ip], aw = A.aw[ip];
+        d4k out;
+#pragma unroll
+        for (int m = 0; m < kVecK; ++m) {
+            const int kc = m * Q + lane;
+            const double ac = carry ? acv[m] : ((acj - atu[kc]) - abu[kc]) / A.max_diag;
+            const double tq = m + 1 < kVecK ? xa[m + 1] : nb.kf;
+            const double bq = m > 0 ? xa[m - 1] : nb.kb;
+            const double ax = ac * xa[m] + ae * xn[m] + aw * xb[m] + an * nb.n[m] + as * nb.s[m] + at[kc] * tq +
+                              ab[kc] * bq;
+            out[m] = xa[m] + (rhs[m] - ax) / ac;
+        }
+        return out;
+    };
+    In nx0 = load0(i0 - kFLag);
+    d4k aca = {1.0, 1.0, 1.0, 1.0}, acb = aca;  // the diagonal at t-1, t-2
+    int cw = 0;
+    for (int t = i0 - kFLag; t < i1 + kFLag; ++t) {
+        d4k z1n, vn, acn;
+        {
+            const double acj = (A.acx[clamp_i(t)] - anu) - asu;
+#pragma unroll
+            for (int m = 0; m < kVecK; ++m) {
+                if (WHICH == 0)
+                    vn[m] = first ? nx0.r[m] : nx0.r[m] + beta * (nx0.v[m] - om * nx0.q[m]);
+                else
+                    vn[m] = nx0.r[m] - alpha * nx0.q[m];
+                const int kc = m * Q + lane;
+                acn[m] = ((acj - atu[kc]) - abu[kc]) / A.max_diag;
+                z1n[m] = vn[m] / acn[m];
+            }
+            if (owned && t >= own0 && t < i1) put(vout, t, vn);
+        }
+        nx0 = load0(t + 1);
+        const double* const prev = lv + (cw ^ 1) * 2 * plane + near;
+        double* const now = lv + cw * 2 * plane + me;
+        const int p1 = t - 1, p2 = t - 2;
+        const d4k z2n = sweep(p1, nbrs(prev), z1b, z1a, z1n, va, aca);
+        if (owned && p2 >= own0 && p2 < i1) put(zout, p2, sweep(p2, nbrs(prev + plane), z2b, z2a, z2n, vb, acb));
+        if (row < G.R) {
+            *(d2a*)now = d2a{z1n[0], z1n[1]};
+            *(d2a*)(now + half) = d2a{z1n[2], z1n[3]};
+            *(d2a*)(now + plane) = d2a{z2n[0], z2n[1]};
+            *(d2a*)(now + plane + half) = d2a{z2n[2], z2n[3]};
+        }
+        __syncthreads();
+        cw ^= 1;
+        z1b = z1a;
+        z1a = z1n;
+        vb = va;
+        va = vn;
+        z2b = z2a;
+        z2a = z2n;
+        if (carry) {
+            acb = aca;
+            aca = acn;
+        }
+    }
+}
+
+// Its split of a grid: every number of j tiles is priced, a block (one per compute unit:
+// its wavefronts fill the VGPRs) taking ni + 2 kFLag steps priced at 1.5 us + 0.3 us per
+// wavefront; no split where fewer than 10 rows fit a block (rows above 304 cells).
+HalfGeom split_pc(const dalm_ctx* ctx) {
+    const Dims& d = ctx->d;
+    const int Q = (d.nz + 3) / 4, most = kPcThreads / Q;
+    HalfGeom best{};
+    double cost = 0;
+    if (most < 2 * kFLag + 4) return best;
+    for (int tj = (d.ny + most - 2 * kFLag - 1) / (most - 2 * kFLag); tj <= d.ny; ++tj) {
+        const int R = (d.ny + tj - 1) / tj + 2 * kFLag;
+        if (R < 2 * kFLag + 4) break;
+        const int waves = (R * Q + 63) / 64;
+        const size_t lds = sizeof(double) * (16 * (size_t)R * (Q + 2) + 16 * (size_t)Q);
+        if (lds > 160 * 1024) continue;
+        for (int rounds = 1; rounds <= 2; ++rounds) {
+            int nch = std::min(rounds * ctx->ncu / tj, (d.nx + 1) / 2);
+            if (nch < 1) continue;
+            const int ni = (d.nx + nch - 1) / nch, blocks = tj * ((d.nx + ni - 1) / ni);
+            const double c = (double)((blocks + ctx->ncu - 1) / ctx->ncu) * (ni + 2 * kFLag) * (1.5 + 0.3 * waves);
+            if (best.R == 0 || c < cost) {
+                cost = c;
+                best = HalfGeom{R, Q, tj, 1, ni, blocks, waves * 64, 0, 0, false, lds};
+            }
+        }
+    }
+    return best;
+}
+
 __global__ void k_zero(long long n, double* __restrict__ a) {
     for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < n;
          e += (long long)gridDim.x * blockDim.x)
@@ -841,6 +1030,10 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
     if (fused) {
         if (const int rz = ensure_fused_z64(ctx)) return rz;
     }
+    // other rows: the update and the sweeps as one kernel as well (k_half_pc: the faster one
+    // at every size measured), p in a pair; rows of other multiples of 256 keep k_jacobi4
+    const HalfGeom pcg = jac && pc_it == 3 && !vec4 ? split_pc(ctx) : HalfGeom{};
+    const bool halves = pcg.R > 0;
     // the fused iteration k writes z_p / z_s into buffer pair k mod kXGroup; its x updates
     // are applied kXGroup at a time, after iterations k = kXGroup - 1 mod kXGroup
     double* PP[kXGroup] = {ctx->pp};
@@ -935,15 +1128,26 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
                                        it_start + k + 1, (const SolveState*)ctx->solve);
                 continue;
             }
-            probe_begin(ctx, DALM_K_PUPDATE);
-            if (vec4)
-                hipLaunchKernelGGL(k_bi_p4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->kp, ctx->q,
-                                   ctx->pp, pc_first, (const SolveState*)ctx->solve);
-            else
-                hipLaunchKernelGGL(k_bi_p, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->kp,
-                                   ctx->q, ctx->pp, pc_first, (const SolveState*)ctx->solve);
-            probe_end(ctx, DALM_K_PUPDATE);
-            double* ppz = precondition(ctx->pp, ctx->tmp, ctx->kp);
+            double *ppz = ctx->pp, *ssz = ctx->ss;
+            const long long k = launched + c;
+            double* const P[2] = {ctx->kp, ctx->tmp};
+            if (halves) {
+                probe_begin(ctx, DALM_K_HALF_P);
+                hipLaunchKernelGGL(k_half_pc<0>, dim3(pcg.blocks), dim3(pcg.threads), pcg.lds, ctx->stream, d, A,
+                                   (const double*)ctx->r, (const double*)P[k & 1], (const double*)ctx->q,
+                                   P[(k + 1) & 1], ppz, pcg, (const SolveState*)ctx->solve);
+                probe_end(ctx, DALM_K_HALF_P);
+            } else {
+                probe_begin(ctx, DALM_K_PUPDATE);
+                if (vec4)
+                    hipLaunchKernelGGL(k_bi_p4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->kp, ctx->q,
+                                       ctx->pp, pc_first, (const SolveState*)ctx->solve);
+                else
+                    hipLaunchKernelGGL(k_bi_p, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->kp,
+                                       ctx->q, ctx->pp, pc_first, (const SolveState*)ctx->solve);
+                probe_end(ctx, DALM_K_PUPDATE);
+                ppz = precondition(ctx->pp, ctx->tmp, ctx->kp);
+            }
             probe_begin(ctx, DALM_K_SPMV);
             if (vec4)
                 hipLaunchKernelGGL(k_bi_spmv4<0>, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A, ppz, ctx->q,
@@ -953,15 +1157,23 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
                                    ctx->q, ctx->r0, ctx->partials, ctx->counter, ctx->solve);
             probe_end(ctx, DALM_K_SPMV);
             if (int rc1 = launch_finalize(ctx, FIN_ALPHA, nb, ctx->solve, nullptr)) return rc1;
-            probe_begin(ctx, DALM_K_SUPDATE);
-            if (vec4)
-                hipLaunchKernelGGL(k_bi_s4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->q, ctx->s,
-                                   ctx->ss, pc_first, (const SolveState*)ctx->solve);
-            else
-                hipLaunchKernelGGL(k_bi_s, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->q,
-                                   ctx->s, ctx->ss, pc_first, (const SolveState*)ctx->solve);
-            probe_end(ctx, DALM_K_SUPDATE);
-            double* ssz = precondition(ctx->ss, ctx->tmp2, ctx->s);
+            if (halves) {
+                probe_begin(ctx, DALM_K_HALF_S);
+                hipLaunchKernelGGL(k_half_pc<1>, dim3(pcg.blocks), dim3(pcg.threads), pcg.lds, ctx->stream, d, A,
+                                   (const double*)ctx->r, (const double*)nullptr, (const double*)ctx->q, ctx->s, ssz,
+                                   pcg, (const SolveState*)ctx->solve);
+                probe_end(ctx, DALM_K_HALF_S);
+            } else {
+                probe_begin(ctx, DALM_K_SUPDATE);
+                if (vec4)
+                    hipLaunchKernelGGL(k_bi_s4, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->q, ctx->s,
+                                       ctx->ss, pc_first, (const SolveState*)ctx->solve);
+                else
+                    hipLaunchKernelGGL(k_bi_s, dim3(ctx->sgrid), dim3(BLOCK), 0, ctx->stream, d, A, ctx->r, ctx->q,
+                                       ctx->s, ctx->ss, pc_first, (const SolveState*)ctx->solve);
+                probe_end(ctx, DALM_K_SUPDATE);
+                ssz = precondition(ctx->ss, ctx->tmp2, ctx->s);
+            }
             probe_begin(ctx, DALM_K_SPMV);
             if (vec4)
                 hipLaunchKernelGGL(k_bi_spmv4<1>, dim3(grid4), dim3(BLOCK), 0, ctx->stream, d, A, ssz, ctx->t,
@@ -1007,6 +1219,7 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
         hipLaunchKernelGGL(k_x_flush, dim3(ctx->grid), dim3(BLOCK), 0, ctx->stream, d, x, pring(last), f);
         LAUNCH_CHECK();
     }
+    if (halves && (done_it & 1)) std::swap(ctx->kp, ctx->tmp);
     if (fused && (done_it & 1)) {
         // after an odd number of iterations the current p and q are the partners
         std::swap(ctx->kp, ctx->tmp);
