@@ -59,9 +59,11 @@ static int ensure_slots(dalm_ctx* ctx, long long n) {
 
 int copy_out(dalm_ctx* ctx, void* const c[3], int nc, bool f32, double* host) {
     const long long total = ctx->L * nc, slot = std::min({kSlot, std::max((total + 3) / 4, kSmall), total});
-    if (total < kSmall) {
+    if (total < kSmall || ensure_slots(ctx, slot) != DALM_OK) {
+        (void)hipGetLastError();
         // no pinned slots: making them takes longer than they save at first (0.71 against 0.34 ms
-        // for six fields of 32x20x20, 2.6 against 2.9 at 64x48x48)
+        // for six fields of 32x20x20, 2.6 against 2.9 at 64x48x48);
+        // nor where the host grants none
         std::vector<double> tmp(ctx->L);
         std::vector<float> tmpf(f32 ? ctx->L : 0);
         for (int q = 0; q < nc; ++q) {
@@ -71,7 +73,6 @@ int copy_out(dalm_ctx* ctx, void* const c[3], int nc, bool f32, double* host) {
         }
         return DALM_OK;
     }
-    if (const int rc = ensure_slots(ctx, slot)) return rc;
     const long long chunks = (total + slot - 1) / slot;
     const auto length = [&](long long n) { return std::min(slot, total - n * slot); };
     const auto pack = [&](long long n) -> int {

@@ -597,7 +597,7 @@ int dalm_upload(dalm_ctx* ctx, int64_t field, const double* host) {
 int dalm_download(dalm_ctx* ctx, int64_t field, double* host) {
     CHECK_CTX();
     if (!host) return DALM_BAD_ARG;
-    void* c[3];
+    void* c[3] = {};
     int nc;
     bool f32;
     TRY(field_ptrs(ctx, field, c, &nc, &f32));
