@@ -136,7 +136,8 @@ PROBE_IDS = {"jacobi": 1, "spmv": 2, "update": 3, "predictor": 4, "sor": 5, "res
 
 
 def fused_rows(mesh, case):
-    """The half-iterations run fused on rows of exactly 256 cells with BiCGStab(Jacobi x3)."""
+    """The whole iteration runs fused on rows of exactly 256 cells with BiCGStab(Jacobi x3)
+    (other rows: the half-iterations, with the r and x update as a pass)."""
     return mesh.interior[2] == 256 and case.method == "BiCG" and case.pc == "Jacobi" and case.pc_it == 3
 FORMS = ("fp64", "mixed")
 
@@ -562,6 +563,8 @@ def main():
         if a.probe == "auto":
             if fused_rows(case.mesh, case):
                 probe = "half_p" if form == "fp64" else "half_p_mixed"
+            elif case.method == "BiCG" and case.pc == "Jacobi" and case.pc_it == 3:
+                probe = "update" if form == "fp64" else "update_mixed"
             else:
                 probe = "jacobi" if form == "fp64" else "jacobi32"
         else:
