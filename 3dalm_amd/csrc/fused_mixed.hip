@@ -30,8 +30,8 @@
 //
 // What bounds it: HBM on rows of 256 cells at 512x256x256 (295 and 230 us a half: 4.1 and
 // 3.5 TB/s of algorithmic bytes, 4.4 and 3.9 with the halos, where a plain copy reaches
-// 4.8); below that the steps' issue and LDS (3.4 and 2.9 us a step of 11 wavefronts at
-// 256x128x128, 48 and 40 us a half, where the five separate kernels took 52 and 49).
+// 4.8); below that the steps' issue and LDS (3.0 and 2.8 us a step of 11 wavefronts at
+// 256x128x128, 42 and 39 us a half, where the separate kernels took 52 and 49).
 //
 // The arithmetic per cell is that of the separate kernels (kg_p4 / kg_s4, kf_jacobi4,
 // kg_spmv4), in their order: FP32 sweeps with FP32 coefficients, the SpMV in FP64 with the
@@ -65,6 +65,7 @@
 #include <algorithm>
 #include <type_traits>
 #include "ctx.h"
+#include "stencil.h"
 
 namespace {
 
@@ -531,10 +532,10 @@ static HalfGeom split_half(const dalm_ctx* ctx) {
         // from kColsFrom cells on chunks and tiles of whole units of the separate kernels, but
         // where those cost a quarter more (at 192x128x384 264 blocks, eight of them in a second
         // round: 5.27 ms a step and 4.26; the pressure's error against 64 bits is 4e-7 in
-        // either); rows of a multiple of 256 have others (col_unit4)
+        // either); rows that the separate kernels take four cells per lane have others (col_unit4)
         double cost, cost_cols;
         best = cheapest_half(ctx, false, &cost);
-        if (ctx->N >= kColsFrom && d.nz % 256) {
+        if (ctx->N >= kColsFrom && !vec4_applies(d)) {
             const HalfGeom c = cheapest_half(ctx, true, &cost_cols);
             if (c.R > 0 && cost_cols <= 1.25 * cost) best = c;
         }
@@ -548,8 +549,8 @@ static HalfGeom split_half(const dalm_ctx* ctx) {
 // The fused path: three Jacobi sweeps on a grid that splits (R > 0).  It is the faster one
 // at every size measured, a step of 10 iterations with the separate kernels and fused:
 // 654 and 569 us at 30x14x16, 678 and 629 at 96x48x48, 806 and 701 at 128x64x64, 939 and 862 at
-// 64x96x128, 1295 and 1048 at 173x101x87, 1993 and 1830 at 256x128x128, 8110 and 6366 at
-// 400x200x190.  Rows too long for a
+// 64x96x128, 1295 and 1048 at 173x101x87, 8110 and 6366 at
+// 400x200x190, and of 12 iterations 2245 and 2058 at 256x128x128.  Rows too long for a
 // block take k tiles, whose halo quads cost more, from kTilesFrom cells on: 639 and 648 at
 // 20x16x700, but 815 and 751 at 60x64x300, 1393 and 1364 at 40x100x600; where the separate
 // kernels' wavefronts fill (rows of whole wavefronts) from twice that: 766 and 775 at

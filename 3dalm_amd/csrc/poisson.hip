@@ -1031,7 +1031,7 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
         if (const int rz = ensure_fused_z64(ctx)) return rz;
     }
     // other rows: the update and the sweeps as one kernel as well (k_half_pc: the faster one
-    // at every size measured), p in a pair; rows of other multiples of 256 keep k_jacobi4
+    // at every size measured), p in a pair; rows of four cells per lane keep k_jacobi4
     const HalfGeom pcg = jac && pc_it == 3 && !vec4 ? split_pc(ctx) : HalfGeom{};
     const bool halves = pcg.R > 0;
     // the fused iteration k writes z_p / z_s into buffer pair k mod kXGroup; its x updates
