@@ -25,6 +25,9 @@
 constexpr int kXGroup = 8;
 constexpr int kXGroupF = 8;
 
+// LDS of a compute unit: a block that asks for more cannot be launched
+constexpr size_t kLdsBytes = 160 * 1024;
+
 // Device-resident scalar state of one Poisson solve (read by every kernel of the
 // solve; written only by the last block of a reduction).
 struct SolveState {
@@ -381,6 +384,10 @@ int zero_device(dalm_ctx* ctx, double* a, long long n);
 // fused half-iterations of the precision form's BiCGStab (fused_mixed.hip)
 // their split of this grid, or null where the fused path does not apply
 const HalfGeom* half_geom(dalm_ctx* ctx, int pc_kind, int pc_it);
+// the splits themselves, host arithmetic on the context's sizes (R = 0: none): the
+// precision form's (fused_mixed.hip) and FP64 rows that are no multiple of 256 (poisson.hip)
+HalfGeom split_half(const dalm_ctx* ctx);
+HalfGeom split_pc(const dalm_ctx* ctx);
 // planes per unit of a fused kernel that runs one block per compute unit over
 // `tiles` j tiles: as many plane chunks as fill the compute units once, chunks of at
 // least 16 planes

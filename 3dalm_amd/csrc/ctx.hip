@@ -9,6 +9,7 @@
 #include <cstring>
 
 #include "ctx.h"
+#include "resident.h"
 
 int dalm_fail(dalm_ctx* ctx, hipError_t e, const char* what, const char* file, int line) {
     if (ctx) {
@@ -363,6 +364,45 @@ int ensure_fused_z64(dalm_ctx* ctx) {
     return DALM_OK;
 }
 
+// whether a context can hold a grid of this padded size
+static bool grid_ok(const int64_t size[3], int64_t gc) {
+    if (gc < 2 || gc > 16) return false;  // the reference asserts gc >= 2 (src/solver.h:615)
+    // 32-bit cell indices: the padded box stays below 2^31 - 2^20 cells (checked
+    // factor by factor, so that no product overflows)
+    constexpr long long kMaxCells = (1LL << 31) - (1LL << 20);
+    for (int a = 0; a < 3; ++a)
+        if (size[a] < 2 * gc + 3 || size[a] >= kMaxCells) return false;
+    long long L = size[0] * size[1];
+    if (L >= kMaxCells) return false;
+    L *= size[2];
+    if (L >= kMaxCells) return false;
+    return true;
+}
+
+// extents, tiles, units and launch sizes of a context of this grid (host only)
+static void size_context(dalm_ctx* ctx, const int64_t size[3], int64_t gc) {
+    ctx->d = make_dims(size, gc);
+    Dims& d = ctx->d;
+    ctx->L = (long long)d.n0 * d.n1 * d.n2;
+    ctx->N = (long long)d.nx * d.ny * d.nz;
+    ctx->grid = cell_grid(d.ntiles);
+    // column units: about 2048 of them, 1 to kMaxColumnPlanes planes each -- small
+    // grids get short columns rather than too few workgroups, large ones long columns
+    // (each unit re-reads a halo plane at either end: 2 per 8 planes cost the
+    // four-cell SpMV and x/r update 4-5 % at 512x256x256 against 2 per 32)
+    {
+        long long per_plane = (long long)d.tj * d.tk;
+        long long ni = (d.nx * per_plane + 2047) / 2048;
+        if (ni < 1) ni = 1;
+        if (ni > kMaxColumnPlanes) ni = kMaxColumnPlanes;
+        if (ni > d.nx) ni = d.nx;
+        d.ni = (int)ni;
+        d.nch = (d.nx + d.ni - 1) / d.ni;
+        d.nunits = (int)(per_plane * d.nch);
+        ctx->sgrid = d.nunits;
+    }
+}
+
 extern "C" {
 
 int dalm_set_device(int64_t device) {
@@ -394,40 +434,14 @@ int dalm_create(dalm_ctx** out, const int64_t size[3], int64_t gc, const double*
                 const double* z, int64_t precision) {
     if (!out || !size || !x || !y || !z) return DALM_BAD_ARG;
     *out = nullptr;
-    if (gc < 2 || gc > 16) return DALM_BAD_ARG;  // the reference asserts gc >= 2 (src/solver.h:615)
-    // 32-bit cell indices: the padded box stays below 2^31 - 2^20 cells (checked
-    // factor by factor, so that no product overflows)
-    constexpr long long kMaxCells = (1LL << 31) - (1LL << 20);
-    for (int a = 0; a < 3; ++a)
-        if (size[a] < 2 * gc + 3 || size[a] >= kMaxCells) return DALM_BAD_ARG;
-    long long L = size[0] * size[1];
-    if (L >= kMaxCells) return DALM_BAD_ARG;
-    L *= size[2];
-    if (L >= kMaxCells) return DALM_BAD_ARG;
+    if (!grid_ok(size, gc)) return DALM_BAD_ARG;
     if (precision != DALM_FP64 && precision != DALM_MIXED) return DALM_BAD_ARG;
 
     dalm_ctx* ctx = new dalm_ctx();
-    ctx->d = make_dims(size, gc);
-    Dims& d = ctx->d;
-    ctx->L = L;
-    ctx->N = (long long)d.nx * d.ny * d.nz;
     ctx->precision = (int)precision;
-    ctx->grid = cell_grid(d.ntiles);
-    // column units: about 2048 of them, 1 to kMaxColumnPlanes planes each -- small
-    // grids get short columns rather than too few workgroups, large ones long columns
-    // (each unit re-reads a halo plane at either end: 2 per 8 planes cost the
-    // four-cell SpMV and x/r update 4-5 % at 512x256x256 against 2 per 32)
-    {
-        long long per_plane = (long long)d.tj * d.tk;
-        long long ni = (d.nx * per_plane + 2047) / 2048;
-        if (ni < 1) ni = 1;
-        if (ni > kMaxColumnPlanes) ni = kMaxColumnPlanes;
-        if (ni > d.nx) ni = d.nx;
-        d.ni = (int)ni;
-        d.nch = (d.nx + d.ni - 1) / d.ni;
-        d.nunits = (int)(per_plane * d.nch);
-        ctx->sgrid = d.nunits;
-    }
+    size_context(ctx, size, gc);
+    Dims& d = ctx->d;
+    const long long L = ctx->L;
 
     ctx->hx.assign(x, x + d.n0);
     ctx->hy.assign(y, y + d.n1);
@@ -946,6 +960,29 @@ int dalm_set_fp32_pass_cap(dalm_ctx* ctx, int64_t n) {
     CHECK_CTX();
     if (n < 0) return DALM_BAD_ARG;
     ctx->fp32_pass_cap = n;
+    return DALM_OK;
+}
+
+int dalm_solver_split(const int64_t size[3], int64_t gc, int64_t ncu, int64_t what, int64_t out[8]) {
+    if (!size || !out || !grid_ok(size, gc) || ncu < 1 || ncu > 4096 || what < DALM_SPLIT_HALVES ||
+        what > DALM_SPLIT_BICGSTAB)
+        return DALM_BAD_ARG;
+    dalm_ctx ctx;  // sizes only: no device work
+    size_context(&ctx, size, gc);
+    ctx.ncu = (int)ncu;
+    std::fill(out, out + 8, 0);
+    if (what == DALM_SPLIT_HALVES || what == DALM_SPLIT_HALVES_MIXED) {
+        const HalfGeom G = what == DALM_SPLIT_HALVES ? split_pc(&ctx) : split_half(&ctx);
+        if (G.R == 0) return DALM_OK;
+        const int64_t v[8] = {G.blocks, G.threads, (int64_t)G.lds, G.R, G.Q, G.tj, G.tk, G.ni};
+        std::copy(v, v + 8, out);
+    } else {
+        const ResShape s = what == DALM_SPLIT_SOR ? res_shape(&ctx, (ctx.d.nz + 1) / 2, 2 * sizeof(double))
+                                                  : res_shape(&ctx, ctx.d.nz, sizeof(double));
+        if (s.blocks == 0) return DALM_OK;
+        const int64_t v[8] = {s.blocks, s.threads, (int64_t)s.lds, s.P, s.nk, s.M, s.rw, 0};
+        std::copy(v, v + 8, out);
+    }
     return DALM_OK;
 }
 

@@ -483,6 +483,9 @@ int fused_planes(const dalm_ctx* ctx, int tiles) {
 // everything around it, chunks of four 63.7, the separate kernels 59.0 to 66.1.
 constexpr long long kTilesFrom = 1LL << 20, kColsFrom = 1LL << 21;
 
+// what block_sum16 keeps in LDS beside half_lds, at most
+constexpr size_t kHalfStatic = 5 * (kHalfThreads / 64) * sizeof(double);
+
 static HalfGeom cheapest_half(const dalm_ctx* ctx, bool cols, double* cost_out) {
     const Dims& d = ctx->d;
     const int NQ = (d.nz + 3) / 4;
@@ -499,6 +502,8 @@ static HalfGeom cheapest_half(const dalm_ctx* ctx, bool cols, double* cost_out) 
             const int R = own + 2 * kLag;
             if (own < 4) break;
             if (own > most - 2 * kLag || (cols && tk > 1 && (Q - 2) % 16)) continue;
+            // short rows: each of a block's many rows costs its pads too (320 B at one quad)
+            if (half_lds(R, Q) + kHalfStatic > kLdsBytes) continue;
             const int waves = (R * Q + 63) / 64;
             const int per_cu = waves <= 6 ? 12 / waves : 1;
             const int slots = ctx->ncu * per_cu;
@@ -522,7 +527,7 @@ static HalfGeom cheapest_half(const dalm_ctx* ctx, bool cols, double* cost_out) 
     return best;
 }
 
-static HalfGeom split_half(const dalm_ctx* ctx) {
+HalfGeom split_half(const dalm_ctx* ctx) {
     const Dims& d = ctx->d;
     HalfGeom best{};
     if (d.nz == 256 && d.ny >= 10) {

@@ -863,35 +863,6 @@ __global__ __launch_bounds__(kPcThreads) void k_half_pc(Dims d, PCoef A, const d
     }
 }
 
-// Its split of a grid: every number of j tiles is priced, a block (one per compute unit:
-// its wavefronts fill the VGPRs) taking ni + 2 kFLag steps priced at 1.5 us + 0.3 us per
-// wavefront; no split where fewer than 10 rows fit a block (rows above 304 cells).
-HalfGeom split_pc(const dalm_ctx* ctx) {
-    const Dims& d = ctx->d;
-    const int Q = (d.nz + 3) / 4, most = kPcThreads / Q;
-    HalfGeom best{};
-    double cost = 0;
-    if (most < 2 * kFLag + 4) return best;
-    for (int tj = (d.ny + most - 2 * kFLag - 1) / (most - 2 * kFLag); tj <= d.ny; ++tj) {
-        const int R = (d.ny + tj - 1) / tj + 2 * kFLag;
-        if (R < 2 * kFLag + 4) break;
-        const int waves = (R * Q + 63) / 64;
-        const size_t lds = sizeof(double) * (16 * (size_t)R * (Q + 2) + 16 * (size_t)Q);
-        if (lds > 160 * 1024) continue;
-        for (int rounds = 1; rounds <= 2; ++rounds) {
-            int nch = std::min(rounds * ctx->ncu / tj, (d.nx + 1) / 2);
-            if (nch < 1) continue;
-            const int ni = (d.nx + nch - 1) / nch, blocks = tj * ((d.nx + ni - 1) / ni);
-            const double c = (double)((blocks + ctx->ncu - 1) / ctx->ncu) * (ni + 2 * kFLag) * (1.5 + 0.3 * waves);
-            if (best.R == 0 || c < cost) {
-                cost = c;
-                best = HalfGeom{R, Q, tj, 1, ni, blocks, waves * 64, 0, 0, false, lds};
-            }
-        }
-    }
-    return best;
-}
-
 __global__ void k_zero(long long n, double* __restrict__ a) {
     for (long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x; e < n;
          e += (long long)gridDim.x * blockDim.x)
@@ -915,6 +886,35 @@ long long next_chunk(long long done_it, long long predicted, long long max_it) {
 }
 
 }  // namespace
+
+// Its split of a grid: every number of j tiles is priced, a block (one per compute unit:
+// its wavefronts fill the VGPRs) taking ni + 2 kFLag steps priced at 1.5 us + 0.3 us per
+// wavefront; no split where fewer than 10 rows fit a block (rows above 304 cells).
+HalfGeom split_pc(const dalm_ctx* ctx) {
+    const Dims& d = ctx->d;
+    const int Q = (d.nz + 3) / 4, most = kPcThreads / Q;
+    HalfGeom best{};
+    double cost = 0;
+    if (most < 2 * kFLag + 4 || vec4_applies(d)) return best;
+    for (int tj = (d.ny + most - 2 * kFLag - 1) / (most - 2 * kFLag); tj <= d.ny; ++tj) {
+        const int R = (d.ny + tj - 1) / tj + 2 * kFLag;
+        if (R < 2 * kFLag + 4) break;
+        const int waves = (R * Q + 63) / 64;
+        const size_t lds = sizeof(double) * (16 * (size_t)R * (Q + 2) + 16 * (size_t)Q);
+        if (lds > kLdsBytes) continue;
+        for (int rounds = 1; rounds <= 2; ++rounds) {
+            int nch = std::min(rounds * ctx->ncu / tj, (d.nx + 1) / 2);
+            if (nch < 1) continue;
+            const int ni = (d.nx + nch - 1) / nch, blocks = tj * ((d.nx + ni - 1) / ni);
+            const double c = (double)((blocks + ctx->ncu - 1) / ctx->ncu) * (ni + 2 * kFLag) * (1.5 + 0.3 * waves);
+            if (best.R == 0 || c < cost) {
+                cost = c;
+                best = HalfGeom{R, Q, tj, 1, ni, blocks, waves * 64, 0, 0, false, lds};
+            }
+        }
+    }
+    return best;
+}
 
 #define LAUNCH_CHECK() HIP_TRY(hipGetLastError())
 
@@ -1032,7 +1032,7 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
     }
     // other rows: the update and the sweeps as one kernel as well (k_half_pc: the faster one
     // at every size measured), p in a pair; rows of four cells per lane keep k_jacobi4
-    const HalfGeom pcg = jac && pc_it == 3 && !vec4 ? split_pc(ctx) : HalfGeom{};
+    const HalfGeom pcg = jac && pc_it == 3 ? split_pc(ctx) : HalfGeom{};
     const bool halves = pcg.R > 0;
     // the fused iteration k writes z_p / z_s into buffer pair k mod kXGroup; its x updates
     // are applied kXGroup at a time, after iterations k = kXGroup - 1 mod kXGroup

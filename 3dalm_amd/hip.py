@@ -129,6 +129,7 @@ def lib():
         "dalm_probe_read": [V, PI64, P],
         "dalm_set_fp32_pass_cap": [V, i64],
         "dalm_last_solve_info": [V, PI64],
+        "dalm_solver_split": [PI64, i64, i64, i64, PI64],
         "dalm_predictor_adj": [V, dbl, dbl],
         "dalm_interpolate_JU_adj": [V],
         "dalm_apply_JUbc_adj": [V],
@@ -161,6 +162,22 @@ def exported_symbols():
     import re
     text = open(hdr).read()
     return sorted(set(re.findall(r"\b(dalm_[a-z0-9_A-Z]+)\s*\(", text)))
+
+
+SPLIT_HALVES, SPLIT_HALVES_MIXED, SPLIT_SOR, SPLIT_BICGSTAB = range(4)
+
+
+def solver_split(interior, what, ncu=256, gc=2):
+    """The split of a grid by the kernels that keep a part of it on chip
+    (dalm_solver_split, host only), or None where they do not apply."""
+    size, out = (i64 * 3)(*(n + 2 * gc for n in interior)), (i64 * 8)()
+    rc = lib().dalm_solver_split(size, gc, ncu, what, out)
+    if rc != OK:
+        raise HipError(f"dalm_solver_split: {STATUS_NAMES.get(rc, rc)}")
+    names = (("blocks", "threads", "lds", "rows", "quads", "tj", "tk", "planes")
+             if what in (SPLIT_HALVES, SPLIT_HALVES_MIXED) else
+             ("blocks", "threads", "lds", "planes", "positions", "per_thread", "rows", "_"))
+    return dict(zip(names, out)) if out[0] else None
 
 
 def ptr(a):

@@ -290,6 +290,16 @@ int dalm_set_fp32_pass_cap(dalm_ctx *ctx, int64_t n);
  * iteration in an FP64 context), out[2] residual replacements (precision form). */
 int dalm_last_solve_info(dalm_ctx *ctx, int64_t out[3]);
 
+/* Host only: how the kernels that keep a part of the grid on chip would split a grid
+ * of this padded size over ncu compute units; out[0] = 0 where they do not apply.
+ * Fused half-iterations of BiCGStab with three Jacobi sweeps (FP64: on rows that are no
+ * multiple of 256; precision form): blocks, threads, LDS bytes, rows and quads of four
+ * cells of a block, j tiles, k tiles, planes per block.  Solves in one launch: blocks,
+ * threads, LDS bytes, planes per block, positions per row (SOR: pairs of cells),
+ * positions per thread, rows per pass of the threads, 0. */
+enum dalm_split { DALM_SPLIT_HALVES = 0, DALM_SPLIT_HALVES_MIXED = 1, DALM_SPLIT_SOR = 2, DALM_SPLIT_BICGSTAB = 3 };
+int dalm_solver_split(const int64_t size[3], int64_t gc, int64_t ncu, int64_t what, int64_t out[8]);
+
 /* ---- whole step ----------------------------------------------------------------- */
 
 /* Start-up pass of Solver::initialize after the fields are filled

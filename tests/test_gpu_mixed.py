@@ -162,11 +162,13 @@ def test_mixed_passes_and_fp64_hand_over(builder, cap):
 
 @pytest.mark.parametrize("interior, iters", [(s, n) for s in ((9, 10, 13), (33, 30, 87), (40, 24, 64), (70, 13, 30),
                                                               (82, 20, 643), (12, 10, 256)) for n in (1, 2, 9)] +
-                         [((131, 130, 125), 2), ((129, 127, 132), 2), ((50, 150, 283), 2)])
+                         [((131, 130, 125), 2), ((129, 127, 132), 2), ((50, 150, 283), 2),
+                          ((500, 512, 3), 2)])
 def test_fused_half_iterations(interior, iters):
     """The fused half-iterations on rows of any length (quads that reach beyond the row,
     rows cut into k tiles, a last j tile and a last plane chunk of fewer cells, rows of 256
-    cells; from two million cells on chunks and tiles of whole units): the pressure after the first iterations of a step against the FP64
+    cells; from two million cells on chunks and tiles of whole units; rows of one quad in
+    blocks of as many rows as their LDS takes): the pressure after the first iterations of a step against the FP64
     oracle's.  An iteration rounds each vector about 16 times to FP32 (2^-24), and
     BiCGStab lets that grow by up to a factor 3 per iteration; a cell, row or update left
     out is off by more than 1e-3.  After 9 iterations one group of eight pressure updates
