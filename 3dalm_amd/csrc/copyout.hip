@@ -44,7 +44,7 @@ __global__ __launch_bounds__(BLOCK) void k_interleave(const T* c0, const T* c1, 
 }  // namespace
 
 static int ensure_slots(dalm_ctx* ctx, long long n) {
-    if (ctx->out_slot >= n) return DALM_OK;
+    if (ctx->out_slot >= n && ctx->may_take(DALM_PATH_COPY_SLOTS)) return DALM_OK;
     if (ctx->out_pin) {
         (void)hipHostFree(ctx->out_pin);
         ctx->out_pin = nullptr;
@@ -52,7 +52,9 @@ static int ensure_slots(dalm_ctx* ctx, long long n) {
     }
     for (hipEvent_t& e : ctx->out_ev)
         if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    HIP_TRY(hipHostMalloc((void**)&ctx->out_pin, 2 * (size_t)n * sizeof(double), hipHostMallocCoherent));
+    HIP_TRY(ctx->may_take(DALM_PATH_COPY_SLOTS)
+                ? hipHostMalloc((void**)&ctx->out_pin, 2 * (size_t)n * sizeof(double), hipHostMallocCoherent)
+                : hipErrorOutOfMemory);
     ctx->out_slot = n;
     return DALM_OK;
 }
@@ -64,6 +66,7 @@ int copy_out(dalm_ctx* ctx, void* const c[3], int nc, bool f32, double* host) {
         // no pinned slots: making them takes longer than they save at first (0.71 against 0.34 ms
         // for six fields of 32x20x20, 2.6 against 2.9 at 64x48x48);
         // nor where the host grants none
+        ++ctx->taken[DALM_PATH_COPY_PLAIN];
         std::vector<double> tmp(ctx->L);
         std::vector<float> tmpf(f32 ? ctx->L : 0);
         for (int q = 0; q < nc; ++q) {
@@ -73,6 +76,7 @@ int copy_out(dalm_ctx* ctx, void* const c[3], int nc, bool f32, double* host) {
         }
         return DALM_OK;
     }
+    ++ctx->taken[DALM_PATH_COPY_SLOTS];
     const long long chunks = (total + slot - 1) / slot;
     const auto length = [&](long long n) { return std::min(slot, total - n * slot); };
     const auto pack = [&](long long n) -> int {

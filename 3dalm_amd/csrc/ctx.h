@@ -274,6 +274,11 @@ struct dalm_ctx {
     bool res_dirty = true, res_off = false;
     int res_spin = 0;
 
+    // ways gone (dalm_paths_taken), and those switched off or on for tests (dalm_set_paths)
+    int64_t taken[DALM_PATHS] = {};
+    int64_t paths_off = 0, paths_on = 0;
+    bool may_take(int path) const { return !((paths_off >> path) & 1); }
+
     // run parameters (dalm_set_params)
     dalm_params prm{};
     bool have_prm = false;

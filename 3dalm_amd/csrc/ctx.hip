@@ -963,25 +963,41 @@ int dalm_set_fp32_pass_cap(dalm_ctx* ctx, int64_t n) {
     return DALM_OK;
 }
 
-int dalm_solver_split(const int64_t size[3], int64_t gc, int64_t ncu, int64_t what, int64_t out[8]) {
+int dalm_paths_taken(dalm_ctx* ctx, int64_t count[DALM_PATHS]) {
+    CHECK_CTX();
+    if (!count) return DALM_BAD_ARG;
+    std::copy(ctx->taken, ctx->taken + DALM_PATHS, count);
+    return DALM_OK;
+}
+
+int dalm_set_paths(dalm_ctx* ctx, int64_t off, int64_t on) {
+    CHECK_CTX();
+    const int64_t can_off = 1 << DALM_PATH_ONE_LAUNCH | 1 << DALM_PATH_HALVES | 1 << DALM_PATH_COPY_SLOTS;
+    if ((off & ~can_off) || (on & ~(int64_t)(1 << DALM_PATH_HALVES)) || (off & on)) return DALM_BAD_ARG;
+    ctx->paths_off = off;
+    ctx->paths_on = on;
+    return DALM_OK;
+}
+
+int dalm_solver_split(const int64_t size[3], int64_t gc, int64_t ncu, int64_t what, int64_t out[9]) {
     if (!size || !out || !grid_ok(size, gc) || ncu < 1 || ncu > 4096 || what < DALM_SPLIT_HALVES ||
         what > DALM_SPLIT_BICGSTAB)
         return DALM_BAD_ARG;
     dalm_ctx ctx;  // sizes only: no device work
     size_context(&ctx, size, gc);
     ctx.ncu = (int)ncu;
-    std::fill(out, out + 8, 0);
+    std::fill(out, out + 9, 0);
     if (what == DALM_SPLIT_HALVES || what == DALM_SPLIT_HALVES_MIXED) {
         const HalfGeom G = what == DALM_SPLIT_HALVES ? split_pc(&ctx) : split_half(&ctx);
         if (G.R == 0) return DALM_OK;
-        const int64_t v[8] = {G.blocks, G.threads, (int64_t)G.lds, G.R, G.Q, G.tj, G.tk, G.ni};
-        std::copy(v, v + 8, out);
+        const int64_t v[9] = {G.blocks, G.threads, (int64_t)G.lds, G.R, G.Q, G.tj, G.tk, G.ni, G.cols};
+        std::copy(v, v + 9, out);
     } else {
         const ResShape s = what == DALM_SPLIT_SOR ? res_shape(&ctx, (ctx.d.nz + 1) / 2, 2 * sizeof(double))
                                                   : res_shape(&ctx, ctx.d.nz, sizeof(double));
         if (s.blocks == 0) return DALM_OK;
-        const int64_t v[8] = {s.blocks, s.threads, (int64_t)s.lds, s.P, s.nk, s.M, s.rw, 0};
-        std::copy(v, v + 8, out);
+        const int64_t v[7] = {s.blocks, s.threads, (int64_t)s.lds, s.P, s.nk, s.M, s.rw};
+        std::copy(v, v + 7, out);
     }
     return DALM_OK;
 }

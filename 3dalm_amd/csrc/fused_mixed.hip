@@ -562,7 +562,7 @@ HalfGeom split_half(const dalm_ctx* ctx) {
 // 64x48x384, 796 and 824 at 60x64x320, 1763 and 1676 at 96x100x320, 1074 and 1077 at 100x80x384
 // and with 12 iterations 5550 and 4212 at 192x128x384.
 const HalfGeom* half_geom(dalm_ctx* ctx, int pc_kind, int pc_it) {
-    if (pc_kind != DALM_PC_JACOBI || pc_it != 3) return nullptr;
+    if (pc_kind != DALM_PC_JACOBI || pc_it != 3 || !ctx->may_take(DALM_PATH_HALVES)) return nullptr;
     if (!ctx->have_half) {
         ctx->half = split_half(ctx);
         ctx->have_half = true;

@@ -958,6 +958,7 @@ int run_sor_on(dalm_ctx* ctx, double* x, const double* b, int slot, double omega
         *err = ctx->h_solve->err;
         return ctx->h_solve->status;
     }
+    ++ctx->taken[DALM_PATH_LAUNCHES];
     const double root_n = sqrt((double)ctx->N);
     hipLaunchKernelGGL(k_state_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->solve, tol, max_it, root_n);
     LAUNCH_CHECK();
@@ -1026,14 +1027,16 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
     // rows of exactly 256 cells with three Jacobi sweeps: the update and the sweeps of
     // each half-iteration are one kernel (k_half_pc4); p and q alternate between a
     // buffer pair (the Jacobi partners, unused on that path)
-    const bool fused = jac && pc_it == 3 && d.nz == 256 && d.ny >= kFOwn;
+    const bool fusable = jac && pc_it == 3 && ctx->may_take(DALM_PATH_HALVES);
+    const bool fused = fusable && d.nz == 256 && d.ny >= kFOwn;
     if (fused) {
         if (const int rz = ensure_fused_z64(ctx)) return rz;
     }
     // other rows: the update and the sweeps as one kernel as well (k_half_pc: the faster one
     // at every size measured), p in a pair; rows of four cells per lane keep k_jacobi4
-    const HalfGeom pcg = jac && pc_it == 3 ? split_pc(ctx) : HalfGeom{};
+    const HalfGeom pcg = fusable ? split_pc(ctx) : HalfGeom{};
     const bool halves = pcg.R > 0;
+    ++ctx->taken[fused || halves ? DALM_PATH_HALVES : DALM_PATH_LAUNCHES];
     // the fused iteration k writes z_p / z_s into buffer pair k mod kXGroup; its x updates
     // are applied kXGroup at a time, after iterations k = kXGroup - 1 mod kXGroup
     double* PP[kXGroup] = {ctx->pp};

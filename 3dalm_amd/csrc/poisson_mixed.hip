@@ -723,6 +723,7 @@ int run_sor_mixed(dalm_ctx* ctx, double omega, long long max_it, double tol, lon
         *err = ctx->h_solve->err;
         return ctx->h_solve->status;
     }
+    ++ctx->taken[DALM_PATH_LAUNCHES];
     hipLaunchKernelGGL(ks_state_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->solve, tol, max_it,
                        sqrt((double)ctx->N), (double)kSorInner);
     LAUNCH_CHECK();
@@ -778,6 +779,7 @@ int run_poisson_mixed(dalm_ctx* ctx, int pc_kind, double pc_omega, int pc_it, lo
     // not use)
     const HalfGeom* split = half_geom(ctx, pc_kind, pc_it);
     const bool halves = split != nullptr;
+    ++ctx->taken[halves ? DALM_PATH_HALVES : DALM_PATH_LAUNCHES];
     const HalfGeom fgeom = halves ? *split : HalfGeom{};
     const int fgrid = fgeom.sums;
     // rows of 256 cells: the p-half also forms r, and x follows every kXGroupF iterations.
@@ -903,7 +905,8 @@ int run_poisson_mixed(dalm_ctx* ctx, int pc_kind, double pc_omega, int pc_it, lo
         bool stalled = false;
         probe_solve_begin(ctx);
         while (launched < max_it - total) {
-            const long long chunk = chunk_for(launched, ctx->prev_it[1], max_it - total);
+            long long chunk = chunk_for(launched, ctx->prev_it[1], max_it - total);
+            if (test_cap > launched && chunk > test_cap - launched) chunk = test_cap - launched;
             for (long long c = 0; c < chunk; ++c) {
                 probe_iteration(ctx, launched + c);
                 if (fused) {

@@ -448,11 +448,13 @@ int res_finish(dalm_ctx* ctx, double* x, bool* ran) {
     if (*flag != 0) {
         // something keeps this context's blocks off the GPU: it does not wait for that again
         ctx->res_off = true;
+        ++ctx->taken[DALM_PATH_GIVEN_UP];
         return DALM_OK;
     }
     hipLaunchKernelGGL(k_res_commit, dim3(ctx->grid), dim3(BLOCK), 0, ctx->stream, ctx->d, x, (const double*)ctx->r);
     HIP_TRY(hipGetLastError());
     *ran = true;
+    ++ctx->taken[DALM_PATH_ONE_LAUNCH];
     return DALM_OK;
 }
 
@@ -460,7 +462,7 @@ int res_finish(dalm_ctx* ctx, double* x, bool* ran) {
 // available to other programs between them), and so does one whose launches are timed.
 constexpr long long kResMaxIterations = 20000;
 bool res_may_run(const dalm_ctx* ctx, long long max_it) {
-    return !ctx->res_off && max_it <= kResMaxIterations && ctx->probe.kernel == 0;
+    return !ctx->res_off && ctx->may_take(DALM_PATH_ONE_LAUNCH) && max_it <= kResMaxIterations && ctx->probe.kernel == 0;
 }
 
 int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long max_it, double tol, bool* ran) {

@@ -129,6 +129,8 @@ def lib():
         "dalm_probe_read": [V, PI64, P],
         "dalm_set_fp32_pass_cap": [V, i64],
         "dalm_last_solve_info": [V, PI64],
+        "dalm_paths_taken": [V, PI64],
+        "dalm_set_paths": [V, i64, i64],
         "dalm_solver_split": [PI64, i64, i64, i64, PI64],
         "dalm_predictor_adj": [V, dbl, dbl],
         "dalm_interpolate_JU_adj": [V],
@@ -164,19 +166,20 @@ def exported_symbols():
     return sorted(set(re.findall(r"\b(dalm_[a-z0-9_A-Z]+)\s*\(", text)))
 
 
+PATHS = ("one_launch", "given_up", "halves", "launches", "copy_slots", "copy_plain")
 SPLIT_HALVES, SPLIT_HALVES_MIXED, SPLIT_SOR, SPLIT_BICGSTAB = range(4)
 
 
 def solver_split(interior, what, ncu=256, gc=2):
     """The split of a grid by the kernels that keep a part of it on chip
     (dalm_solver_split, host only), or None where they do not apply."""
-    size, out = (i64 * 3)(*(n + 2 * gc for n in interior)), (i64 * 8)()
+    size, out = (i64 * 3)(*(n + 2 * gc for n in interior)), (i64 * 9)()
     rc = lib().dalm_solver_split(size, gc, ncu, what, out)
     if rc != OK:
         raise HipError(f"dalm_solver_split: {STATUS_NAMES.get(rc, rc)}")
-    names = (("blocks", "threads", "lds", "rows", "quads", "tj", "tk", "planes")
+    names = (("blocks", "threads", "lds", "rows", "quads", "tj", "tk", "planes", "unit_sums")
              if what in (SPLIT_HALVES, SPLIT_HALVES_MIXED) else
-             ("blocks", "threads", "lds", "planes", "positions", "per_thread", "rows", "_"))
+             ("blocks", "threads", "lds", "planes", "positions", "per_thread", "rows"))
     return dict(zip(names, out)) if out[0] else None
 
 
@@ -390,6 +393,17 @@ class Context:
     def set_fp32_pass_cap(self, n):
         """Testing aid of the precision form: FP32 passes end after n iterations."""
         self.check(self.L.dalm_set_fp32_pass_cap(self.h, int(n)), "set_fp32_pass_cap")
+
+    def paths_taken(self):
+        """How often each way of a solve or a copy (PATHS) was gone so far."""
+        out = (i64 * len(PATHS))()
+        self.check(self.L.dalm_paths_taken(self.h, out), "paths_taken")
+        return dict(zip(PATHS, out))
+
+    def set_paths(self, off=(), on=()):
+        """Testing aid: ways (of PATHS) to do without, and to go wherever they can."""
+        mask = [sum(1 << PATHS.index(w) for w in ways) for ways in (off, on)]
+        self.check(self.L.dalm_set_paths(self.h, *mask), "set_paths")
 
     # ---- discrete adjoint (bars are the *_b fields)
     def predictor_adj(self, Re, dt):

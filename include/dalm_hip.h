@@ -290,15 +290,35 @@ int dalm_set_fp32_pass_cap(dalm_ctx *ctx, int64_t n);
  * iteration in an FP64 context), out[2] residual replacements (precision form). */
 int dalm_last_solve_info(dalm_ctx *ctx, int64_t out[3]);
 
+/* The ways a solve or a copy of a whole field can go.  dalm_paths_taken: how often each
+ * was gone since dalm_create.  A solve of the precision form that goes on in FP64 counts
+ * for each; DALM_PATH_GIVEN_UP counts launches of DALM_PATH_ONE_LAUNCH whose blocks
+ * waited for each other too long (other programs kept some of them off the GPU): the
+ * solve then runs another way, and so do the context's later ones. */
+enum dalm_path {
+    DALM_PATH_ONE_LAUNCH = 0, /* small grids: the whole solve in one launch      */
+    DALM_PATH_GIVEN_UP = 1,
+    DALM_PATH_HALVES = 2,     /* BiCGStab with fused half-iterations (Jacobi x3) */
+    DALM_PATH_LAUNCHES = 3,   /* a launch per sweep, product and update          */
+    DALM_PATH_COPY_SLOTS = 4, /* dalm_download through pinned slots              */
+    DALM_PATH_COPY_PLAIN = 5, /* dalm_download component by component            */
+    DALM_PATHS = 6
+};
+int dalm_paths_taken(dalm_ctx *ctx, int64_t count[DALM_PATHS]);
+/* Testing aid: `off`, bits 1 << dalm_path of ways that the context is to do without
+ * (one launch, halves; pinned slots: as if none could be allocated); `on`, of ways to go
+ * wherever they can, not only where they are the faster ones (halves).  0, 0: the default. */
+int dalm_set_paths(dalm_ctx *ctx, int64_t off, int64_t on);
 /* Host only: how the kernels that keep a part of the grid on chip would split a grid
  * of this padded size over ncu compute units; out[0] = 0 where they do not apply.
  * Fused half-iterations of BiCGStab with three Jacobi sweeps (FP64: on rows that are no
  * multiple of 256; precision form): blocks, threads, LDS bytes, rows and quads of four
- * cells of a block, j tiles, k tiles, planes per block.  Solves in one launch: blocks,
- * threads, LDS bytes, planes per block, positions per row (SOR: pairs of cells),
- * positions per thread, rows per pass of the threads, 0. */
+ * cells of a block, j tiles, k tiles, planes per block, 1 where the dot products are
+ * summed in the order of the separate kernels.  Solves in one launch: blocks, threads,
+ * LDS bytes, planes per block, positions per row (SOR: pairs of cells), positions per
+ * thread, rows per pass of the threads, 0, 0. */
 enum dalm_split { DALM_SPLIT_HALVES = 0, DALM_SPLIT_HALVES_MIXED = 1, DALM_SPLIT_SOR = 2, DALM_SPLIT_BICGSTAB = 3 };
-int dalm_solver_split(const int64_t size[3], int64_t gc, int64_t ncu, int64_t what, int64_t out[8]);
+int dalm_solver_split(const int64_t size[3], int64_t gc, int64_t ncu, int64_t what, int64_t out[9]);
 
 /* ---- whole step ----------------------------------------------------------------- */
 

@@ -11,9 +11,10 @@ hip = importlib.import_module("3dalm_amd.hip")
 pytestmark = pytest.mark.gpu
 
 
-def _round_trip(interior, precision, seed):
+def _round_trip(interior, precision, seed, off=(), way=None):
     mesh = cases.case_c1(*interior, steps=1).mesh
     ctx = hip.Context(mesh, precision)
+    ctx.set_paths(off)
     try:
         rng = np.random.default_rng(seed)
         for _ in range(2):  # the second pass finds the slots there
@@ -22,17 +23,25 @@ def _round_trip(interior, precision, seed):
                 ctx.upload(name, a)
                 want = a.astype(np.float32).astype(np.float64) if precision == hip.MIXED and name != "p" else a
                 assert np.array_equal(ctx.download(name), want), name
+        assert way is None or ctx.paths_taken()[way] == 6, ctx.paths_taken()
     finally:
         ctx.close()
 
 
 # one and three components below and above the plain copies' 2^18 values, one slot, slots of
 # a quarter, full slots with a remainder
-@pytest.mark.parametrize("interior", [(20, 12, 12), (70, 33, 31), (97, 49, 46), (150, 90, 77)])
+@pytest.mark.parametrize("interior, way", [((20, 12, 12), "copy_plain"), ((70, 33, 31), None),
+                                           ((97, 49, 46), "copy_slots"), ((150, 90, 77), "copy_slots")])
 @pytest.mark.parametrize("precision", [hip.FP64, hip.MIXED])
-def test_copy_out(interior, precision):
+def test_copy_out(interior, way, precision):
     print(f"[copy out {interior} {precision}]", flush=True)
-    _round_trip(interior, precision, 7)
+    _round_trip(interior, precision, 7, way=way)
+
+
+@pytest.mark.parametrize("precision", [hip.FP64, hip.MIXED])
+def test_copy_out_without_pinned_memory(precision):
+    """Where the host grants no pinned memory the plain copies bring the same bytes."""
+    _round_trip((97, 49, 46), precision, 7, off=("copy_slots",), way="copy_plain")
 
 
 def test_copy_out_from_two_threads():

@@ -1,5 +1,6 @@
 """FP64 BiCGStab with three Jacobi sweeps, whose half-iterations are fused on rows of any
-length, against the oracle: the first iterations, to the rounding of the dot products."""
+length, against the oracle: the first iterations, to the rounding of the dot products;
+and against the separate kernels, bit for bit."""
 import importlib
 
 import numpy as np
@@ -18,12 +19,12 @@ def ok():
     return po.Kernels("oracle")
 
 
-# rows of a quad and a cell; rows of whole quads; a last j tile and a last chunk of fewer
-# cells; rows of three and two cells over; rows near the longest a block takes; on grids that
-# the one-launch solver would take, that is told to give up (a limit of one poll)
-@pytest.mark.parametrize("shape", [(7, 6, 5), (40, 20, 24), (65, 33, 31), (33, 47, 62), (20, 12, 303), (70, 97, 85)])
-def test_first_iterations(ok, shape, monkeypatch):
-    monkeypatch.setenv("DALM_RESIDENT_SPIN", "1")
+# rows of a quad and a cell, of one quad; rows of whole quads; a last j tile and a last chunk
+# of fewer cells; rows of three and two cells over; rows near the longest a block takes
+# (small grids take another way unless told to)
+@pytest.mark.parametrize("shape", [(7, 6, 5), (9, 30, 3), (40, 20, 24), (65, 33, 31), (33, 47, 62), (20, 12, 303),
+                                   (20, 13, 383), (70, 97, 85)])
+def test_first_iterations(ok, shape):
     print(f"[half pc {shape}]", flush=True)
     mesh = small_mesh(*shape, 1.2)
     g = po.make_grid(mesh)
@@ -32,8 +33,11 @@ def test_first_iterations(ok, shape, monkeypatch):
     m = interior_mask(mesh)
     p = rand_field(mesh, 71, 1, 0.1)
     b = rand_field(mesh, 72, 1, 1.0) * m
-    c = hip.Context(mesh)
+    c, sep = hip.Context(mesh), hip.Context(mesh)
+    c.set_paths(("one_launch",), ("halves",))
+    sep.set_paths(("one_launch", "halves"))
     c.upload("b", b)
+    sep.upload("b", b)
     work = np.zeros(9 * mesh.L)
     it, err = po.C.c_int64(), po.C.c_double()
     # a dot product's rounding is 1e-16 of it, an iteration lets a difference grow by up to 10
@@ -47,4 +51,9 @@ def test_first_iterations(ok, shape, monkeypatch):
         print(f"  {n} iterations: pressure {d:.2e}", flush=True)
         assert git == it.value == n and st == hip.NONCONVERGED and d <= bound
         assert np.array_equal(c.download("p")[~m], p[~m])
+        sep.upload("p", p)
+        assert sep.run_bicgstab(hip.PC_JACOBI, 1.0, 3, n, 0.0) == (git, gerr, st)
+        assert np.array_equal(c.download("p"), sep.download("p"))
+    assert c.paths_taken()["halves"] == sep.paths_taken()["launches"] == 3
     c.close()
+    sep.close()

@@ -127,14 +127,17 @@ def test_mixed_sor_method(interior, tol):
         s.close()
 
 
-@pytest.mark.parametrize("builder,cap", [(lambda: cases.case_c2(48, 24, 24, steps=3, ap_per_blade=8), 40)] +
-                         [(lambda: _rows256(), cap) for cap in (40, 41, 42, 43)])
-def test_mixed_passes_and_fp64_hand_over(builder, cap):
+@pytest.mark.parametrize("on", [(), ("halves",)])
+@pytest.mark.parametrize("builder,cap", [(build, cap) for cap in (40, 41, 42, 43) for build in (
+    lambda: cases.case_c2(48, 24, 24, steps=3, ap_per_blade=8), lambda: _rows256())])
+def test_mixed_passes_and_fp64_hand_over(builder, cap, on):
     """The precision form's recovery paths: with every FP32 pass cut short after
-    40 iterations (dalm_set_fp32_pass_cap), a pass that ends far
+    40 to 43 iterations (dalm_set_fp32_pass_cap), a pass that ends far
     above the tolerance is restarted from the true residual and one that ends
     within 30x of it is handed over to FP64; every solve must still end on the
-    true residual with the step matching the FP64 oracle.  Also with rows of 256
+    true residual with the step matching the FP64 oracle.  After an odd number of
+    iterations p and q are in the other buffers of their pairs, in the FP32 halves
+    and (switched on for this size) in the FP64 ones that go on from them.  Also with rows of 256
     cells (the fused half-iterations, whose pressure updates are applied eight
     iterations' at a time: caps of 40 to 43 iterations end passes with different
     numbers of them outstanding)."""
@@ -145,34 +148,46 @@ def test_mixed_passes_and_fp64_hand_over(builder, cap):
     o = po.OracleSolver(case)
     s = solver.Solver(case, hip.MIXED)
     s.ctx.set_fp32_pass_cap(cap)
+    s.ctx.set_paths((), on)
     try:
+        in_fp64 = 0
         for _ in range(3):
             so, sm = o.step(), s.step()
-            print(f"step {sm['step']}: it {sm['it']} err {sm['err']:.3e}", flush=True)
+            print(f"step {sm['step']}: it {sm['it']} err {sm['err']:.3e} {s.ctx.last_solve_info()}", flush=True)
             assert sm["status"] == hip.OK, sm
             assert sm["err"] <= case.tol
             assert sm["it"] > cap  # the cut-short pass was followed by more work
+            in_fp64 += s.ctx.last_solve_info()[1]
             assert abs(sm["power"][0] - case.sites[0].rot_speed * so["torque"][0]) <= \
                 1e-3 * abs(case.sites[0].rot_speed * so["torque"][0])
+        assert in_fp64 > 0
         m = interior_mask(case.mesh)
         assert rel_l2(s.field("U")[m], o.field("U")[m]) <= 1e-4
     finally:
         s.close()
 
 
+# grids whose dot products are summed by whole units, with their k tiles
+UNIT_SUMS = {(131, 130, 125): 1, (129, 127, 132): 1, (81, 154, 184): 3, (71, 67, 442): 7}
+
+
 @pytest.mark.parametrize("interior, iters", [(s, n) for s in ((9, 10, 13), (33, 30, 87), (40, 24, 64), (70, 13, 30),
                                                               (82, 20, 643), (12, 10, 256)) for n in (1, 2, 9)] +
                          [((131, 130, 125), 2), ((129, 127, 132), 2), ((50, 150, 283), 2),
-                          ((500, 512, 3), 2)])
+                          ((500, 512, 3), 2), ((81, 154, 184), 2), ((71, 67, 442), 2)])
 def test_fused_half_iterations(interior, iters):
     """The fused half-iterations on rows of any length (quads that reach beyond the row,
     rows cut into k tiles, a last j tile and a last plane chunk of fewer cells, rows of 256
-    cells; from two million cells on chunks and tiles of whole units; rows of one quad in
+    cells; from two million cells on chunks and tiles of whole units, with one and several
+    k tiles; rows of one quad in
     blocks of as many rows as their LDS takes): the pressure after the first iterations of a step against the FP64
     oracle's.  An iteration rounds each vector about 16 times to FP32 (2^-24), and
     BiCGStab lets that grow by up to a factor 3 per iteration; a cell, row or update left
     out is off by more than 1e-3.  After 9 iterations one group of eight pressure updates
     has been applied and one is outstanding."""
+    if interior in UNIT_SUMS:
+        split = hip.solver_split(interior, hip.SPLIT_HALVES_MIXED)
+        assert split["unit_sums"] and split["tk"] == UNIT_SUMS[interior], split
     case = cases.case_c1(*interior, steps=1)
     case.method, case.pc, case.pc_it, case.max_it, case.tol = "BiCG", "Jacobi", 3, iters, 0.0
     print(f"[fused halves {interior} {iters} iterations]", flush=True)
@@ -186,5 +201,28 @@ def test_fused_half_iterations(interior, iters):
         assert d <= 16 * 2.0 ** -24 * 3.0 ** (iters - 1) * 4
         outside = s.field("p")[~m]
         assert np.all(np.isfinite(outside))
+        assert s.ctx.paths_taken()["halves"] == 1
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("interior", [(9, 10, 13), (33, 30, 87), (70, 13, 30), (12, 10, 256), (8, 3, 40)])
+@pytest.mark.parametrize("sweeps, iters", [(3, 1), (3, 2), (3, 9), (1, 2), (2, 2), (4, 5)])
+def test_separate_kernels(interior, sweeps, iters):
+    """The update, sweeps and product as kernels of their own (any number of sweeps but
+    three, rows of fewer than four cells along j, three sweeps switched off), as
+    test_fused_half_iterations: the same roundings, a few more with a fourth sweep."""
+    case = cases.case_c1(*interior, steps=1)
+    case.method, case.pc, case.pc_it, case.max_it, case.tol = "BiCG", "Jacobi", sweeps, iters, 0.0
+    print(f"[separate kernels {interior} {sweeps} sweeps {iters} iterations]", flush=True)
+    o, s = po.OracleSolver(case), solver.Solver(case, hip.MIXED)
+    s.ctx.set_paths(("halves",))
+    try:
+        so, sm = o.step(), s.step()
+        assert sm["it"] == so["it"] == iters and s.ctx.paths_taken()["launches"] == 1
+        m = interior_mask(case.mesh)
+        d = rel_l2(s.field("p")[m], o.field("p")[m])
+        print(f"  pressure {d:.2e}", flush=True)
+        assert d <= 16 * 2.0 ** -24 * 3.0 ** (iters - 1) * 4
     finally:
         s.close()

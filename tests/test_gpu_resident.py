@@ -1,8 +1,10 @@
 """The one-launch solvers of small grids (csrc/resident.hip) against the oracle: SOR
 iterates bit for bit, BiCGStab's first iterations to the rounding of its dot products
 and its converged solution, over splits into one and several slabs, odd row lengths,
-a last slab of fewer planes, and a stop by the tolerance in mid-solve."""
+a last slab of fewer planes, and a stop by the tolerance in mid-solve.  Every test
+states how the grid is split and asserts that its solves ran in one launch."""
 import importlib
+import threading
 
 import numpy as np
 import pytest
@@ -33,15 +35,31 @@ def _problem(ok, shape):
     return mesh, g, A, p, b, c
 
 
-# one slab; 64 slabs of one plane; 33 slabs of two planes, the last of one, odd rows;
-# more rows than threads hold at once (several positions per thread); rows longer than
-# two wavefronts
-SHAPES = [(7, 6, 5), (3, 12, 33), (64, 10, 9), (65, 33, 31), (20, 64, 64), (130, 20, 150)]
+# shape, blocks, planes of a block, positions per thread: one slab and several, a last one
+# of fewer planes, 64 of one plane, odd rows, rows longer than two wavefronts
+SOR_SHAPES = [((7, 6, 5), 1, 7, 1), ((3, 12, 33), 1, 3, 1), ((5, 3, 194), 1, 5, 3), ((14, 55, 3), 1, 14, 4),
+              ((64, 10, 9), 64, 1, 1), ((65, 33, 31), 33, 2, 2), ((4, 15, 203), 4, 1, 3), ((20, 64, 64), 20, 1, 4),
+              ((67, 3, 263), 34, 2, 1), ((3, 11, 269), 3, 1, 4)]
+BI_SHAPES = [((7, 6, 5), 1, 7, 1), ((3, 12, 33), 1, 3, 2), ((3, 13, 39), 1, 3, 3), ((19, 27, 3), 1, 19, 4),
+             ((64, 10, 9), 64, 1, 1), ((105, 4, 5), 53, 2, 1), ((65, 19, 27), 33, 2, 2), ((4, 39, 39), 4, 1, 3),
+             ((65, 8, 97), 33, 2, 4), ((71, 4, 131), 36, 2, 2)]
 
 
-@pytest.mark.parametrize("shape", SHAPES)
-def test_sor_bits(ok, shape):
+def _split_is(shape, what, blocks, planes, per_thread):
+    s = hip.solver_split(shape, what)
+    assert (s["blocks"], s["planes"], s["per_thread"]) == (blocks, planes, per_thread), s
+
+
+def _ran(c, **counts):
+    """The solves went these ways and no other."""
+    got = c.paths_taken()
+    assert {k: v for k, v in got.items() if v and not k.startswith("copy")} == counts, got
+
+
+@pytest.mark.parametrize("shape, blocks, planes, per_thread", SOR_SHAPES)
+def test_sor_bits(ok, shape, blocks, planes, per_thread):
     print(f"[resident sor {shape}]", flush=True)
+    _split_is(shape, hip.SPLIT_SOR, blocks, planes, per_thread)
     mesh, g, A, p, b, c = _problem(ok, shape)
     x, r = p.copy(), np.zeros(mesh.L)
     it, err = po.C.c_int64(), po.C.c_double()
@@ -59,13 +77,15 @@ def test_sor_bits(ok, shape):
     got = c.run_sor(1.3, 500, tol)
     assert got[0] == it.value < 500 and got[2] == hip.OK
     assert np.array_equal(c.download("p"), x)
+    _ran(c, one_launch=2)
     c.close()
 
 
 @pytest.mark.parametrize("pc", [hip.PC_JACOBI, hip.PC_SOR])
-@pytest.mark.parametrize("shape", SHAPES)
-def test_bicgstab(ok, shape, pc):
+@pytest.mark.parametrize("shape, blocks, planes, per_thread", BI_SHAPES)
+def test_bicgstab(ok, shape, blocks, planes, per_thread, pc):
     print(f"[resident bicgstab {shape} pc {pc}]", flush=True)
+    _split_is(shape, hip.SPLIT_BICGSTAB, blocks, planes, per_thread)
     mesh, g, A, p, b, c = _problem(ok, shape)
     m = interior_mask(mesh)
     lib = po.lib("oracle")[0]
@@ -85,7 +105,37 @@ def test_bicgstab(ok, shape, pc):
         else:  # both within 1e-13 of the same solution
             assert st == hip.OK and gerr <= 1e-13 and d <= 1e-10
         assert np.array_equal(c.download("p")[~m], p[~m])
+    _ran(c, one_launch=2)
     c.close()
+
+
+def test_two_contexts_at_once(ok):
+    """Solves of two contexts in one launch each, from two threads, over and over: the
+    oracle's iterates in both."""
+    bad = []
+
+    def work(shape):
+        try:
+            mesh, g, A, p, b, c = _problem(ok, shape)
+            x, r = p.copy(), np.zeros(mesh.L)
+            it, err = po.C.c_int64(), po.C.c_double()
+            po.lib("oracle")[0].or_run_sor(po.C.byref(g), po.ptr(A), po.ptr(x), po.ptr(b), po.ptr(r), 1.3,
+                                           po.C.byref(it), 60, po.C.byref(err), 0.0)
+            for _ in range(20):
+                c.upload("p", p)
+                c.run_sor(1.3, 60, 0.0)
+                assert np.array_equal(c.download("p"), x)
+            _ran(c, one_launch=20)
+            c.close()
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            bad.append(e)
+
+    ts = [threading.Thread(target=work, args=(s,)) for s in ((65, 33, 31), (20, 64, 64))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad
 
 
 def test_breakdown_and_nonfinite():
@@ -103,6 +153,7 @@ def test_breakdown_and_nonfinite():
     c.upload("p", np.zeros(mesh.L))
     it, err, st = c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, 50, 1e-8)
     assert it == 1 and st == hip.NONFINITE
+    _ran(c, one_launch=3)
     c.close()
 
 
@@ -119,20 +170,25 @@ def test_falls_back_when_a_wait_ends(ok, monkeypatch):
                                        po.C.byref(err), 0.0)
         got = c.run_sor(1.3, n, 0.0)
         assert got[0] == n and np.array_equal(c.download("p"), x)
+    _ran(c, given_up=1, launches=2)
     c.close()
 
 
-@pytest.mark.parametrize("shape", [(7, 6, 5), (64, 10, 9), (65, 33, 31), (20, 64, 64)])
-def test_sor_mixed(shape):
-    """The precision form's SOR of one step against the FP64 oracle's: after the same
+@pytest.mark.parametrize("way", ["one_launch", "launches"])
+@pytest.mark.parametrize("shape", [(7, 6, 5), (64, 10, 9), (65, 33, 31), (4, 15, 203), (20, 64, 64), (67, 3, 263)])
+def test_sor_mixed(shape, way):
+    """The precision form's SOR of one step, in one launch and with a launch per sweep
+    (as on larger grids), against the FP64 oracle's: after the same
     number of iterations (a multiple of 8) the pressure and the residual differ by the
     FP32 rounding of the corrections, 2^-24 of each (allowed: ten of them), and by that of
     the FP32 predictor in b."""
     cases, solver = importlib.import_module("3dalm_amd.cases"), importlib.import_module("3dalm_amd.solver")
-    print(f"[resident sor mixed {shape}]", flush=True)
+    print(f"[sor mixed {shape} {way}]", flush=True)
+    off = ("one_launch",) if way == "launches" else ()
     case = cases.case_c1(*shape, steps=1)
     case.max_it, case.tol = 24, 0.0
     o, s = po.OracleSolver(case), solver.Solver(case, hip.MIXED)
+    s.ctx.set_paths(off)
     try:
         so, sm = o.step(), s.step()
         assert sm["it"] == so["it"] == 24
@@ -140,10 +196,13 @@ def test_sor_mixed(shape):
         d = rel_l2(s.field("p")[m], o.field("p")[m])
         print(f"  pressure {d:.2e}, err {sm['err']:.6e} against {so['err']:.6e}", flush=True)
         assert d <= 10 * 2.0 ** -24 * 10 and abs(sm["err"] - so["err"]) <= 1e-5 * so["err"]
+        _ran(s.ctx, **{way: 1})
         case.max_it, case.tol = 2000, 0.5 * so["err"]
         s2 = solver.Solver(case, hip.MIXED)
+        s2.ctx.set_paths(off)
         st = s2.step()
         assert st["it"] % 8 == 0 and st["it"] < 2000 and st["err"] <= case.tol
+        _ran(s2.ctx, **{way: 1})
         s2.close()
     finally:
         s.close()
