@@ -887,6 +887,22 @@ long long next_chunk(long long done_it, long long predicted, long long max_it) {
 
 }  // namespace
 
+// Whether the two kernels of an iteration take less time than the six they replace (two
+// updates, four sweeps): those take 34 us and 25 us per million cells in whole tiles, while
+// the vectors stay in the last-level cache; k_half_pc two times 3.0 us + 0.125 us per
+// wavefront for each of its steps and rounds, however few the blocks are.  Fitted to 160 sizes
+// from 10^4 to 2 10^7 cells that do not fit one launch; with it no size is more than 3 %
+// slower than they are.  Steps of 16 iterations with the separate kernels and
+// fused: 869 and 1208 us at 20x12x383, 1119 and 1321 at 30x24x349 (left to the separate
+// ones), 1999 and 2042 the other way round at 64x64x303.  From two million cells on the fused
+// ones were the faster at every size measured (1.01 to 1.5 times).
+static bool halves_pay(const dalm_ctx* ctx, const HalfGeom& G) {
+    if (G.R == 0 || ((ctx->paths_on >> DALM_PATH_HALVES) & 1) || ctx->N >= (1LL << 21)) return true;
+    const int waves = G.threads / 64, rounds = (G.blocks + ctx->ncu - 1) / ctx->ncu;
+    const double padded = 1e-6 * BLOCK * (double)ctx->d.ntiles;
+    return rounds * (G.ni + 2 * kFLag) * (6.0 + 0.25 * waves) < 34.0 + 25.0 * padded;
+}
+
 // Its split of a grid: every number of j tiles is priced, a block (one per compute unit:
 // its wavefronts fill the VGPRs) taking ni + 2 kFLag steps priced at 1.5 us + 0.3 us per
 // wavefront; no split where fewer than 10 rows fit a block (rows above 304 cells).
@@ -1032,9 +1048,10 @@ int run_bicgstab_on(dalm_ctx* ctx, double* x, const double* b, int slot, int pc_
     if (fused) {
         if (const int rz = ensure_fused_z64(ctx)) return rz;
     }
-    // other rows: the update and the sweeps as one kernel as well (k_half_pc: the faster one
-    // at every size measured), p in a pair; rows of four cells per lane keep k_jacobi4
-    const HalfGeom pcg = fusable ? split_pc(ctx) : HalfGeom{};
+    // other rows: the update and the sweeps as one kernel as well (k_half_pc) where that is
+    // faster, p in a pair; rows of four cells per lane keep k_jacobi4
+    const HalfGeom split = fusable ? split_pc(ctx) : HalfGeom{};
+    const HalfGeom pcg = halves_pay(ctx, split) ? split : HalfGeom{};
     const bool halves = pcg.R > 0;
     ++ctx->taken[fused || halves ? DALM_PATH_HALVES : DALM_PATH_LAUNCHES];
     // the fused iteration k writes z_p / z_s into buffer pair k mod kXGroup; its x updates

@@ -311,8 +311,9 @@ int dalm_paths_taken(dalm_ctx *ctx, int64_t count[DALM_PATHS]);
 int dalm_set_paths(dalm_ctx *ctx, int64_t off, int64_t on);
 /* Host only: how the kernels that keep a part of the grid on chip would split a grid
  * of this padded size over ncu compute units; out[0] = 0 where they do not apply.
- * Fused half-iterations of BiCGStab with three Jacobi sweeps (FP64: on rows that are no
- * multiple of 256; precision form): blocks, threads, LDS bytes, rows and quads of four
+ * Fused half-iterations of BiCGStab with three Jacobi sweeps (FP64: on rows that do not
+ * take the four-cell kernels, where the separate kernels are not faster; precision
+ * form): blocks, threads, LDS bytes, rows and quads of four
  * cells of a block, j tiles, k tiles, planes per block, 1 where the dot products are
  * summed in the order of the separate kernels.  Solves in one launch: blocks, threads,
  * LDS bytes, planes per block, positions per row (SOR: pairs of cells), positions per

@@ -57,3 +57,15 @@ def test_first_iterations(ok, shape):
     assert c.paths_taken()["halves"] == sep.paths_taken()["launches"] == 3
     c.close()
     sep.close()
+
+
+# a block's steps cost more than the launches saved where the blocks are few and wide
+@pytest.mark.parametrize("shape, way", [((20, 12, 383), "launches"), ((30, 24, 349), "launches"), ((6, 14, 141), "launches"),
+                                        ((4, 106, 53), "launches"), ((100, 98, 16), "halves"), ((39, 98, 78), "halves")])
+def test_way_of_small_grids(shape, way):
+    mesh = small_mesh(*shape, 1.2)
+    c = hip.Context(mesh)
+    c.upload("b", rand_field(mesh, 72, 1, 1.0) * interior_mask(mesh))
+    c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, 2, 0.0)
+    assert c.paths_taken()[way] == 1, c.paths_taken()
+    c.close()
