@@ -888,19 +888,20 @@ long long next_chunk(long long done_it, long long predicted, long long max_it) {
 }  // namespace
 
 // Whether the two kernels of an iteration take less time than the six they replace (two
-// updates, four sweeps): those take 34 us and 25 us per million cells in whole tiles, while
-// the vectors stay in the last-level cache; k_half_pc two times 3.0 us + 0.125 us per
-// wavefront for each of its steps and rounds, however few the blocks are.  Fitted to 160 sizes
-// from 10^4 to 2 10^7 cells that do not fit one launch; with it no size is more than 3 %
-// slower than they are.  Steps of 16 iterations with the separate kernels and
-// fused: 869 and 1208 us at 20x12x383, 1119 and 1321 at 30x24x349 (left to the separate
-// ones), 1999 and 2042 the other way round at 64x64x303.  From two million cells on the fused
-// ones were the faster at every size measured (1.01 to 1.5 times).
+// updates, four sweeps): with the vectors in the last-level cache those take 22 us (beyond
+// two launches) and 35 us per million cells in whole tiles, k_half_pc two times 2 us +
+// 0.18 us per wavefront for each of its steps and rounds, however few the blocks are.  Fitted
+// to 165 sizes of 10^4 to 2 10^6 cells that do not fit one launch: the choice costs at most
+// 5 % of a step against the better one, 0.1 % in the mean.  Steps of 16 iterations, separate
+// and fused: 801 and 886 us at 4x123x24, 869 and 1208 at 20x12x383, 1119 and 1321 at
+// 30x24x349; 1037 and 1025 at 82x41x35, 1253 and 1215 at 96x64x64, 1999 and 2042 the other way
+// round at 64x64x303.  From two million cells on the fused ones were the faster at every size
+// measured (1.01 to 1.5 times).
 static bool halves_pay(const dalm_ctx* ctx, const HalfGeom& G) {
     if (G.R == 0 || ((ctx->paths_on >> DALM_PATH_HALVES) & 1) || ctx->N >= (1LL << 21)) return true;
     const int waves = G.threads / 64, rounds = (G.blocks + ctx->ncu - 1) / ctx->ncu;
     const double padded = 1e-6 * BLOCK * (double)ctx->d.ntiles;
-    return rounds * (G.ni + 2 * kFLag) * (6.0 + 0.25 * waves) < 34.0 + 25.0 * padded;
+    return rounds * (G.ni + 2 * kFLag) * (4.0 + 0.35 * waves) < 22.0 + 35.0 * padded;
 }
 
 // Its split of a grid: every number of j tiles is priced, a block (one per compute unit:

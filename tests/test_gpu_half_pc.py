@@ -61,7 +61,8 @@ def test_first_iterations(ok, shape):
 
 # a block's steps cost more than the launches saved where the blocks are few and wide
 @pytest.mark.parametrize("shape, way", [((20, 12, 383), "launches"), ((30, 24, 349), "launches"), ((6, 14, 141), "launches"),
-                                        ((4, 106, 53), "launches"), ((100, 98, 16), "halves"), ((39, 98, 78), "halves")])
+                                        ((4, 106, 53), "launches"), ((100, 98, 16), "halves"), ((39, 98, 78), "halves"),
+                                        ((290, 28, 33), "halves"), ((96, 64, 64), "halves")])
 def test_way_of_small_grids(shape, way):
     mesh = small_mesh(*shape, 1.2)
     c = hip.Context(mesh)
