@@ -490,7 +490,8 @@ int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long m
 int res_bicgstab(dalm_ctx* ctx, double* x, const double* b, int pc_kind, double pc_omega, int pc_it, long long max_it,
                  double tol, bool* ran) {
     *ran = false;
-    if (!res_may_run(ctx, max_it) || pc_it < 1) return DALM_OK;
+    // a cap of no iterations (an adjoint solve's) leaves x as it is: this kernel does one at least
+    if (!res_may_run(ctx, max_it) || pc_it < 1 || max_it < 1) return DALM_OK;
     ResShape s = res_shape(ctx, ctx->d.nz, sizeof(double));
     if (s.blocks == 0) return DALM_OK;
     if (int rc = res_prepare(ctx, s)) return rc;

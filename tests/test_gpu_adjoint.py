@@ -175,6 +175,24 @@ def test_poisson_adj(mesh, ok, method, pc):
     assert abs(lhs - rhs) <= tol * abs(lhs), (lhs, rhs)
 
 
+@pytest.mark.parametrize("method,pc,its", [("BiCG", "Jacobi", 0), ("BiCG", "SOR", 0), ("SOR", "Jacobi", 1)])
+@pytest.mark.parametrize("max_it", [0, -3])
+def test_poisson_adj_without_iterations(mesh, method, pc, its, max_it):
+    """A cap below one iteration: BiCGStab runs none and SOR one, in one launch or not."""
+    case = cases.case_c1(6, 5, 5)
+    case.mesh = mesh
+    case.method, case.pc, case.pc_it, case.pc_omega, case.omega = method, pc, 2, 1.1, 1.4
+    got = []
+    for off in ((), ("one_launch",)):
+        c = ctx_with(mesh, p_b=rand_field(mesh, 62, 1, 1.0) * interior_mask(mesh))
+        c.set_params(solver.params_for(case))
+        c.set_paths(off)
+        n, _ = c.poisson_adj(1e-13, max_it)
+        assert n == its
+        got.append(c.download("b_b"))
+    assert np.array_equal(*got)
+
+
 def test_alm_adj(ok):
     case = cases.case_adjoint_small(14, 12, 12, ap_per_blade=5)
     m = case.mesh
