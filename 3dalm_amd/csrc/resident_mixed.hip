@@ -11,6 +11,26 @@
 
 namespace {
 
+// Whether a ghost cell that a block's residual reads holds a value that is not finite.  Their
+// coefficients are zero, so finite ones need no reading (nor registers: with the slab loaded
+// whole, 64x48x48 took 5.24 instead of 5.02 ms), but zero times an infinity is no number, and
+// the solve ends on it as with a launch per sweep.
+template <int M>
+__device__ __forceinline__ bool ghosts_not_finite(const Dims& d, const ResThread<M>& t, const double* __restrict__ x) {
+    const int g = d.gc;
+    bool bad = false;
+    const auto see = [&](int i, int j, int k) { bad |= !(fabs(x[d.at(g + i, g + j, g + k)]) < HUGE_VAL); };
+    for (int e = threadIdx.x; e < t.planes * d.ny; e += blockDim.x)
+        for (int k : {-1, d.nz}) see(t.first + e / d.ny, e % d.ny, k);
+    for (int e = threadIdx.x; e < t.planes * d.nz; e += blockDim.x)
+        for (int j : {-1, d.ny}) see(t.first + e / d.nz, j, e % d.nz);
+    for (int e = threadIdx.x; e < d.ny * d.nz; e += blockDim.x) {
+        if (!t.has_l) see(-1, e / d.nz, e % d.nz);
+        if (!t.has_r) see(d.nx, e / d.nz, e % d.nz);
+    }
+    return bad;
+}
+
 template <int M>
 __global__ __launch_bounds__(res_threads(M)) void k_res_sor_mixed(Dims d, PCoef A, PCoefF Af, ResShape s,
                                                                   const double* __restrict__ x, const double* b,
@@ -20,8 +40,12 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_sor_mixed(Dims d, PCoef 
     extern __shared__ __align__(16) double slab[];  // the residual's x, then the sweeps' e (as floats)
     float* const eslab = (float*)slab;
     __shared__ ResSync sh;
+    __shared__ int ghost;
     if (threadIdx.x < 2) sh.bad[threadIdx.x] = 0;
+    if (threadIdx.x == 0) ghost = 0;
+    __syncthreads();
     ResThread<M> t = res_thread<M>(d, s);
+    if (ghosts_not_finite(d, t, x)) ghost = 1;
     const int g = d.gc;
     const int plane = s.pj * s.pk, half = (s.P + 2) * plane;
     double xv[2][M];
@@ -97,7 +121,7 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_sor_mixed(Dims d, PCoef 
             res_take<double, M>(d, s, t, sh, slab + c * half, keep(c));
         }
         if (!res_barrier(sh, t)) return;
-        double v[1] = {0.0};
+        double v[1] = {it == 0 && ghost ? (double)NAN : 0.0};
         // once in `inner` iterations the FP64 operator and b are read again instead of held
         // beside the sweeps' values; the empty statement keeps the compiler from doing that
         // ahead of the loop (the registers it took spilled: 7.8 ms a solve)

@@ -206,3 +206,32 @@ def test_sor_mixed(shape, way):
         s2.close()
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("off", [(), ("one_launch",)])
+@pytest.mark.parametrize("shape", [(7, 6, 5), (64, 10, 9), (65, 33, 31), (12, 8, 8)])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_sor_mixed_ghost_pressure(shape, value, off):
+    """A pressure that is not finite in a ghost cell next to the interior ends the
+    precision form's SOR as non-finite (its zero coefficient times it is no number), in
+    one launch as with a launch per sweep; in an edge of the box no cell reads it."""
+    cases, solver = importlib.import_module("3dalm_amd.cases"), importlib.import_module("3dalm_amd.solver")
+    print(f"[resident sor mixed ghost {shape} {value}]", flush=True)
+    case = cases.case_c1(*shape, steps=1)
+    case.max_it, case.tol = 16, 0.0
+    g = case.mesh.gc
+    n = [q + 2 * g for q in shape]
+    mid = [g + q // 2 for q in shape]
+    ghosts = [(i, *mid[1:]) for i in (g - 1, n[0] - g)] + [(mid[0], j, mid[2]) for j in (g - 1, n[1] - g)] + \
+        [(*mid[:2], k) for k in (g - 1, n[2] - g)]
+    for ghost, want in [(q, hip.NONFINITE) for q in ghosts] + [((g - 1, g - 1, mid[2]), hip.NONCONVERGED)]:
+        s = solver.Solver(case, hip.MIXED)
+        s.ctx.set_paths(off)
+        p = np.zeros(n)
+        p[ghost] = value
+        s.ctx.upload("p", p.reshape(-1))
+        try:
+            status = s.step()["status"]
+        finally:
+            s.close()
+        assert status == want, (ghost, status)
