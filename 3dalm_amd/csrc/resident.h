@@ -12,7 +12,8 @@
 // and stores kEmpty back.  The value is its own arrival flag, so no fence orders it
 // against a separate flag, and every access is a relaxed agent-scope atomic, which is
 // coherent across the XCDs' L2s.  kEmpty is a signalling NaN: arithmetic never produces
-// one (it returns quiet NaNs), so no computed value can look empty.  Measured: 1.0 us per
+// one (it returns quiet NaNs), so no computed value can look empty (a value that is
+// published uncomputed is quieted first).  Measured: 1.0 us per
 // exchange of 64 words between neighbours and 1.45 us for 1024 words each way, 1.35 us
 // for a value from each of 64 blocks to all of them (a counter barrier costs 1.37 us
 // and carries no data).

@@ -71,7 +71,9 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_sor_mixed(Dims d, PCoef 
             const int k = in ? 2 * t.k + (c ^ o) : 0;
             const bool cell = in && k < d.nz;
             has[c] |= (unsigned)cell << m;
-            xv[c][m] = cell ? x[d.at(i, j, g + k)] : 0.0;
+            // quieted: x is published as it came, and a signalling NaN of the caller's could be
+            // the mark of an empty slot
+            xv[c][m] = cell ? __builtin_canonicalize(x[d.at(i, j, g + k)]) : 0.0;
             const int kc = cell ? g + k : g;
             acf[c][m] = (((Af.acx[i] - Af.anu[j]) - Af.asu[j]) - Af.atu[kc]) - Af.abu[kc];
             rcf[c][m] = __builtin_amdgcn_rcpf(acf[c][m]);

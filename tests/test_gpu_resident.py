@@ -235,3 +235,23 @@ def test_sor_mixed_ghost_pressure(shape, value, off):
         finally:
             s.close()
         assert status == want, (ghost, status)
+
+
+@pytest.mark.parametrize("method", ["SOR mixed", "SOR", "BiCG"])
+def test_pressure_like_an_empty_slot(method):
+    """A pressure whose bits are the mark of an empty exchange slot: the solve is
+    non-finite, and no block waits for the value."""
+    cases, solver = importlib.import_module("3dalm_amd.cases"), importlib.import_module("3dalm_amd.solver")
+    print(f"[resident empty mark {method}]", flush=True)
+    case = cases.case_c1(64, 10, 9, steps=1)
+    case.method, case.pc, case.max_it, case.tol = method.split()[0], "Jacobi", 16, 0.0
+    g = case.mesh.gc
+    p = np.zeros([n + 2 * g for n in (64, 10, 9)])
+    p.view(np.uint64)[g + 20, g + 3, g + 4] = 0x7FF4DEADBEEF0001
+    s = solver.Solver(case, hip.MIXED if method.endswith("mixed") else hip.FP64)
+    try:
+        s.ctx.upload("p", p.reshape(-1))
+        assert s.step()["status"] == hip.NONFINITE
+        _ran(s.ctx, one_launch=1)
+    finally:
+        s.close()
