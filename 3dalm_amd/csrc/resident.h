@@ -337,8 +337,9 @@ __device__ __forceinline__ bool res_sum(const double (&v)[NV], const ResShape& s
 ResShape res_shape(const dalm_ctx* ctx, int lanes, size_t bytes);
 // allocate and empty the exchange slots on first use (sets ctx->res_off without room)
 int res_prepare(dalm_ctx* ctx, ResShape& s);
-// whether this context may run a resident solve of up to max_it iterations now
-bool res_may_run(const dalm_ctx* ctx, long long max_it);
+// whether this context may run a resident solve of up to max_it iterations of so many
+// exchanges now
+bool res_may_run(const dalm_ctx* ctx, long long max_it, long long exchanges);
 // wait for the launch, read its SolveState and copy its result, in ctx->r, to the
 // interior of x; *ran is false when the launch was aborted (x is then as it was)
 int res_finish(dalm_ctx* ctx, double* x, bool* ran);

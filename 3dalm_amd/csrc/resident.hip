@@ -458,16 +458,19 @@ int res_finish(dalm_ctx* ctx, double* x, bool* ran) {
     return DALM_OK;
 }
 
-// A solve that may run longer than this keeps the launches per sweep (the GPU stays
-// available to other programs between them), and so does one whose launches are timed.
-constexpr long long kResMaxIterations = 20000;
-bool res_may_run(const dalm_ctx* ctx, long long max_it) {
-    return !ctx->res_off && ctx->may_take(DALM_PATH_ONE_LAUNCH) && max_it <= kResMaxIterations && ctx->probe.kernel == 0;
+// A solve that may take more exchanges than this keeps the launches per sweep (the GPU stays
+// available to other programs between them), and so does one whose launches are timed: at
+// 1.2 to 2.6 us each a launch ends after about a second at most, whatever its cap of
+// iterations and the sweeps of each (20000 iterations with up to five SOR sweeps fit).
+constexpr long long kResMaxExchanges = 1LL << 19;
+bool res_may_run(const dalm_ctx* ctx, long long max_it, long long exchanges) {
+    return !ctx->res_off && ctx->may_take(DALM_PATH_ONE_LAUNCH) && ctx->probe.kernel == 0 &&
+           max_it <= kResMaxExchanges / exchanges;
 }
 
 int res_sor(dalm_ctx* ctx, double* x, const double* b, double omega, long long max_it, double tol, bool* ran) {
     *ran = false;
-    if (!res_may_run(ctx, max_it)) return DALM_OK;
+    if (!res_may_run(ctx, max_it, 2)) return DALM_OK;
     ResShape s = res_shape(ctx, (ctx->d.nz + 1) / 2, 2 * sizeof(double));
     if (s.blocks == 0) return DALM_OK;
     if (int rc = res_prepare(ctx, s)) return rc;
@@ -491,7 +494,9 @@ int res_bicgstab(dalm_ctx* ctx, double* x, const double* b, int pc_kind, double 
                  double tol, bool* ran) {
     *ran = false;
     // a cap of no iterations (an adjoint solve's) leaves x as it is: this kernel does one at least
-    if (!res_may_run(ctx, max_it) || pc_it < 1 || max_it < 1) return DALM_OK;
+    if (pc_it < 1 || max_it < 1) return DALM_OK;
+    // each half-iteration's sweeps (two colours in SOR), and three sums
+    if (!res_may_run(ctx, max_it, 2LL * pc_it * (pc_kind == DALM_PC_JACOBI ? 1 : 2) + 3)) return DALM_OK;
     ResShape s = res_shape(ctx, ctx->d.nz, sizeof(double));
     if (s.blocks == 0) return DALM_OK;
     if (int rc = res_prepare(ctx, s)) return rc;

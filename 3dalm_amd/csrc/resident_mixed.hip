@@ -196,7 +196,7 @@ __global__ __launch_bounds__(res_threads(M)) void k_res_sor_mixed(Dims d, PCoef 
 
 int res_sor_mixed(dalm_ctx* ctx, double omega, int inner, long long max_it, double tol, bool* ran) {
     *ran = false;
-    if (!res_may_run(ctx, max_it)) return DALM_OK;
+    if (!res_may_run(ctx, max_it, 3)) return DALM_OK;  // two colours, and the refinement's three in `inner`
     ResShape s = res_shape(ctx, (ctx->d.nz + 1) / 2, 2 * sizeof(double));
     if (s.blocks == 0) return DALM_OK;
     if (int rc = res_prepare(ctx, s)) return rc;

@@ -255,3 +255,17 @@ def test_pressure_like_an_empty_slot(method):
         _ran(s.ctx, one_launch=1)
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("solve, way", [
+    (lambda c: c.run_sor(1.3, 20000, 1.0), "one_launch"), (lambda c: c.run_sor(1.3, 300000, 1.0), "launches"),
+    (lambda c: c.run_bicgstab(hip.PC_SOR, 1.1, 5, 20000, 1.0), "one_launch"),
+    (lambda c: c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, 20001, 1.0), "one_launch"),
+    (lambda c: c.run_bicgstab(hip.PC_SOR, 1.1, 60, 20000, 1.0), "launches"),
+    (lambda c: c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, 2**62, 1.0), "launches")])
+def test_way_of_long_solves(ok, solve, way):
+    """The work that a solve may take at most decides, not its cap of iterations alone."""
+    mesh, g, A, p, b, c = _problem(ok, (12, 9, 10))
+    solve(c)
+    _ran(c, **{way: 1})
+    c.close()
