@@ -23,6 +23,7 @@ def _round_trip(interior, precision, seed, off=(), way=None):
                 ctx.upload(name, a)
                 want = a.astype(np.float32).astype(np.float64) if precision == hip.MIXED and name != "p" else a
                 assert np.array_equal(ctx.download(name), want), name
+        assert ctx.L.dalm_last_error(ctx.h) == b""
         assert way is None or ctx.paths_taken()[way] == 6, ctx.paths_taken()
     finally:
         ctx.close()
