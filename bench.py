@@ -80,13 +80,12 @@ HBM_PEAK_GBS = 8000.0
 # per-kernel HBM traffic of this workload from rocprofv3 FETCH_SIZE / WRITE_SIZE runs
 # (3dalm_amd/profile_summary.py traffic --json; the command is in the .md beside it)
 TRAFFIC_JSON = os.path.join(ROOT, "profiles", "hbm_traffic_alm_512x256x256.json")
-# the kernels behind each probe on rows of a multiple of 256 interior cells (the
-# headline grid), where the iteration kernels run four cells per lane
+# the kernels behind each probe on rows of 256 interior cells (the headline grid), where
+# the iteration kernels run four cells per lane and the half-iterations fused
 PROBE_KERNEL = {"jacobi": "k_jacobi4", "jacobi32": "kf_jacobi4", "spmv": "k_bi_spmv4<0>", "update": "k_bi_xr4<0>",
                 "pupdate": "k_bi_p4", "supdate": "k_bi_s4", "predictor": "k_predictor",
                 "spmv_mixed": "kg_spmv4<0>", "update_mixed": "kg_xr4", "pupdate_mixed": "kg_p4",
                 "supdate_mixed": "kg_s4",
-                # rows of exactly 256 cells: the fused half-iterations
                 "half_p_mixed": "kg_half4<0>", "half_s_mixed": "kg_half4<1>",
                 "half_p": "k_half_pc4<0>", "half_s": "k_half_pc4<1>"}
 
@@ -96,8 +95,7 @@ PROBE_BYTES = {
     "jacobi": 24,     # read z_in, v; write z_out
     "spmv": 24,       # read z, a1 (r0 or s); write y
     # read s, t, r0, write r (k_bi_xr4<0>: the fused iteration's x updates are applied
-    # eight at a time by k_x_group4, 144 B; 64 B with x on rows that do not take the
-    # fused iteration)
+    # eight at a time by k_x_group4, 144 B)
     "update": 32,
     "pupdate": 40,    # read r, p, q; write p, z
     "supdate": 32,    # read r, q; write s, z
@@ -119,6 +117,9 @@ PROBE_BYTES = {
     "half_p": 40,        # read r, p, q; write p, z3 (FP64)
     "half_s": 32,        # read r, q; write s, z3 (FP64)
 }
+# on other rows r and x are updated in a pass after the s-half: that pass moves x and both z
+# too (k_bi_xr, k_bi_xr4<1>), and the precision form's halves neither r nor <r0, s>
+PROBE_BYTES_OTHER = {**PROBE_BYTES, "update": 64, "half_p_mixed": 28, "half_s_mixed": 20}
 # algorithmic bytes per interior cell of one whole step: the fixed kernels (predictor,
 # flux + right-hand side, projection, post with div stored) and one BiCGStab(Jacobi 3)
 # iteration, plus the solve's start (residual and shadow residual)
@@ -130,6 +131,9 @@ STEP_BYTES = {"fp64": {"fixed": 104 + 48 + 32 + 104 + 64, "per_it": 280, "per_so
 # + 10 (the x updates of eight iterations every eighth time, 80 B)
 STEP_BYTES_FUSED = {"fp64": {"fixed": 104 + 48 + 32 + 104 + 64, "per_it": 170, "per_solve": 32},
                     "mixed": {"fixed": 64 + 44 + 80 + 48, "per_it": 70, "per_solve": 28}}
+# other rows with fused half-iterations: FP64 40 + 24 + 32 + 24 + 64, precision form 28 + 20
+# + 40 (the update of r and x)
+STEP_BYTES_HALVES = {"fp64": {**STEP_BYTES["fp64"], "per_it": 184}, "mixed": {**STEP_BYTES["mixed"], "per_it": 88}}
 PROBE_IDS = {"jacobi": 1, "spmv": 2, "update": 3, "predictor": 4, "sor": 5, "resnorm": 6, "pupdate": 7,
              "supdate": 8, "jacobi32": 9, "spmv_mixed": 10, "update_mixed": 11, "pupdate_mixed": 12,
              "supdate_mixed": 13, "half_p_mixed": 16, "half_s_mixed": 17, "half_p": 18, "half_s": 19}
@@ -139,6 +143,18 @@ def fused_rows(mesh, case):
     """The whole iteration runs fused on rows of exactly 256 cells with BiCGStab(Jacobi x3)
     (other rows: the half-iterations, with the r and x update as a pass)."""
     return mesh.interior[2] == 256 and case.method == "BiCG" and case.pc == "Jacobi" and case.pc_it == 3
+
+
+def probe_bytes(probe, rows256):
+    """Algorithmic bytes per interior cell of a launch of the probed kernel."""
+    return (PROBE_BYTES if rows256 else PROBE_BYTES_OTHER)[probe]
+
+
+def step_bytes(rows256, halves):
+    """The table of a step's bytes by the way its solves went (`halves`: fused)."""
+    return STEP_BYTES_FUSED if rows256 and halves else STEP_BYTES_HALVES if halves else STEP_BYTES
+
+
 FORMS = ("fp64", "mixed")
 
 
@@ -192,7 +208,7 @@ def run_form(case, precision, steps, warmup, probe, form, keep_fields=False):
         res = {"seconds": t1 - t0, "it_mean": float(np.mean(its)), "it64_mean": float(np.mean(it64)), "it": its,
                "avg_div_max": float(np.max(divs)), "avg_div_last": float(divs[-1]),
                "power_last": power[-1] if power else None,
-               "window": [warmup + 1, warmup + steps]}
+               "window": [warmup + 1, warmup + steps], "halves": s.ctx.paths_taken()["halves"] > 0}
         if probe:
             n, ms = C.c_int64(), C.c_double()
             s.ctx.check(s.ctx.L.dalm_probe_read(s.ctx.h, C.byref(n), C.byref(ms)), "probe_read")
@@ -589,7 +605,7 @@ def main():
             return None
         pr = res["probe"]
         mean_s = pr["total_ms"] / pr["launches"] / 1e3
-        bytes_per_launch = PROBE_BYTES[pr["kernel"]] * N
+        bytes_per_launch = probe_bytes(pr["kernel"], fused) * N
         ach = bytes_per_launch / mean_s / 1e9
         traffic = None
         try:
@@ -678,7 +694,7 @@ def main():
         """whole-step algorithmic bytes (fixed + per iteration x iterations) over the
         time per step (the ALM projection's box and the precision form's residual
         replacements are left out; its FP64 iterations are counted at FP64 bytes)"""
-        table = STEP_BYTES_FUSED if fused else STEP_BYTES
+        table = step_bytes(fused, r["halves"])
         b = table[form]
         if form == "mixed":
             per_it = (b["per_it"] * (r["it_mean"] - r["it64_mean"]) + table["fp64"]["per_it"] * r["it64_mean"])
