@@ -31,7 +31,7 @@
 // What bounds it: HBM on rows of 256 cells at 512x256x256 (295 and 230 us a half: 4.1 and
 // 3.5 TB/s of algorithmic bytes, 4.4 and 3.9 with the halos, where a plain copy reaches
 // 4.8); below that the steps' issue and LDS (3.0 and 2.8 us a step of 11 wavefronts at
-// 256x128x128, 42 and 39 us a half, where the separate kernels took 52 and 49).
+// 256x128x128, 41 and 38 us a half, where the separate kernels took 52 and 49).
 //
 // The arithmetic per cell is that of the separate kernels (kg_p4 / kg_s4, kf_jacobi4,
 // kg_spmv4), in their order: FP32 sweeps with FP32 coefficients, the SpMV in FP64 with the
@@ -82,11 +82,7 @@ typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 //   lv[2][3][R][4 Q + 2 kPad]  the new plane of each stencil input (z1, z2, z3), in two
 //       alternating copies: a step reads the copy the previous step wrote and writes the
 //       other, so one barrier per step orders both (101 of the CU's 160 KB at R Q = 1024)
-//   FP64 k coefficients (SpMV) at, ab, atu, abu [4][Q] each, a lane's four cells Q apart: at
-//       consecutive places the lanes' 16-byte reads, 32 bytes apart, meet in the same LDS
-//       banks (256x128x128 64 / 60 us a half, 55 / 49 apart; where HBM bounds the kernel,
-//       rows of 256 cells, half as many reads are 2 % faster all the same), FP32 ones
-//       (sweeps) [Q][4],
+//   k coefficients at, ab, atu, abu [Q][4] each, FP64 (SpMV) and FP32 (sweeps)
 //   FP64 j coefficients an, as, anu, asu of each row
 __host__ __device__ inline int half_row_len(int Q) { return 4 * Q + 2 * kPad; }
 __host__ __device__ inline size_t half_lds(int R, int Q) {
@@ -237,11 +233,10 @@ __global__ __launch_bounds__(MODE == 2 ? kHalfThreads : kHalfThreadsAny) void kg
     for (int t = threadIdx.x; t < nk; t += blockDim.x) {
         const int k = kbase + t;
         const bool in = k >= g && k < g + d.nz;
-        const int td = UNI ? t : (t & 3) * G.Q + (t >> 2);
-        atd[td] = in ? A.at[k] : 0.0;
-        abd[td] = in ? A.ab[k] : 0.0;
-        atud[td] = in ? A.atu[k] : 1.0;
-        abud[td] = in ? A.abu[k] : 0.0;
+        atd[t] = in ? A.at[k] : 0.0;
+        abd[t] = in ? A.ab[k] : 0.0;
+        atud[t] = in ? A.atu[k] : 1.0;
+        abud[t] = in ? A.abu[k] : 0.0;
         atf[t] = in ? Af.at[k] : 0.f;
         abf[t] = in ? Af.ab[k] : 0.f;
         atuf[t] = in ? Af.atu[k] : 1.f;
@@ -291,7 +286,6 @@ __global__ __launch_bounds__(MODE == 2 ? kHalfThreads : kHalfThreadsAny) void kg
     const int rr = row == 0 ? 1 : (row >= G.R - 1 ? G.R - 2 : row);
     const int me = row * len + kPad + 4 * lane, near = rr * len + kPad + 4 * lane;
     const int lk = 4 * lane;
-    const auto kc = [&](int q) { return UNI ? lk + q : q * G.Q + lane; };
 
     // one step at plane t with L = 0, 1, 2 stencil levels (the pipeline's fill) or 3 (and
     // the SpMV).  (The loop unrolled by two, to rename the pipeline registers instead of
@@ -370,7 +364,7 @@ __global__ __launch_bounds__(MODE == 2 ? kHalfThreads : kHalfThreadsAny) void kg
                     f4 y;
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const double au = (acj - atud[kc(q)]) - abud[kc(q)];
+                        const double au = (acj - atud[lk + q]) - abud[lk + q];
                         double ac = au * inv_md;
                         if (!UNI) ac = fma(fma(-ac, A.max_diag, au), inv_md, ac);  // rounded as au / max_diag
                         const double tq = q + 1 < 4 ? (double)z3a[q + 1] : (double)nb.kf;
@@ -380,8 +374,8 @@ __global__ __launch_bounds__(MODE == 2 ? kHalfThreads : kHalfThreadsAny) void kg
                         yv = fma(aw, (double)z3b[q], yv);
                         yv = fma(and_, (double)nb.n[q], yv);
                         yv = fma(asd, (double)nb.s[q], yv);
-                        yv = fma(atd[kc(q)], tq, yv);
-                        yv = fma(abd[kc(q)], bq, yv);
+                        yv = fma(atd[lk + q], tq, yv);
+                        yv = fma(abd[lk + q], bq, yv);
                         const float yf = (float)yv;
                         y[q] = yf;
                         const double ys = (double)yf;
@@ -477,8 +471,9 @@ int fused_planes(const dalm_ctx* ctx, int tiles) {
 // 16 planes.  Otherwise every number of k and j tiles is priced: a block takes
 // ni + 2 kLag steps of 1.5 us + 0.2 us per wavefront on its compute unit (measured at
 // 10 to 16 wavefronts; both sides of the halos' trade: a thinner chunk or tile recomputes
-// more).  At 256x128x128 8 j tiles of 22 rows and chunks of 8 planes are chosen (53 / 48 us
-// a half); 5 tiles of 32 rows took 55 / 49, two k tiles 59 / 51.  Small grids are left with
+// more).  At 256x128x128 8 j tiles of 22 rows and chunks of 8 planes are chosen (41 and 38 us
+// a half); 4 j tiles of 38 rows in two k tiles took 9 and 8 % more, 8 tiles of 22 rows in
+// two 25 %.  Small grids are left with
 // the steps: chunks of two planes (8 steps) take 57.8 us an iteration at 64x32x32 with
 // everything around it, chunks of four 63.7, the separate kernels 59.0 to 66.1.
 constexpr long long kTilesFrom = 1LL << 20, kColsFrom = 1LL << 21;
