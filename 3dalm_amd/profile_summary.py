@@ -53,7 +53,7 @@ ALGO_BYTES = {
     "k_bi_xr4<0>": 32, "k_bi_xr4<1>": 64, "k_x_group4": 144,
     "kf_jacobi4": 12, "kg_spmv4<0>": 12, "kg_spmv4<1>": 12, "kg_p4": 20, "kg_s4": 16, "kg_xr4": 40,
     # fused half-iterations (Jacobi x3): rows of 256 cells, with r formed in the p-half; others
-    "kg_half4<0>": 36, "kg_half4<1>": 24, "k_half_pc4<0>": 40, "k_half_pc4<1>": 32,
+    "k_half_pc4<0>": 40, "k_half_pc4<1>": 32,
     "kg_half4<0, 2, false>": 36, "kg_half4<1, 2, false>": 24, "k_half_pc<0>": 40, "k_half_pc<1>": 32,
     **{f"kg_half4<{w}, {m}, {c}>": b for w, b in ((0, 28), (1, 20)) for m in (0, 1) for c in ("false", "true")},
     # the fused iteration's x updates of eight iterations (working launches)

@@ -86,7 +86,7 @@ PROBE_KERNEL = {"jacobi": "k_jacobi4", "jacobi32": "kf_jacobi4", "spmv": "k_bi_s
                 "pupdate": "k_bi_p4", "supdate": "k_bi_s4", "predictor": "k_predictor",
                 "spmv_mixed": "kg_spmv4<0>", "update_mixed": "kg_xr4", "pupdate_mixed": "kg_p4",
                 "supdate_mixed": "kg_s4",
-                "half_p_mixed": "kg_half4<0>", "half_s_mixed": "kg_half4<1>",
+                "half_p_mixed": "kg_half4<0, 2, false>", "half_s_mixed": "kg_half4<1, 2, false>",
                 "half_p": "k_half_pc4<0>", "half_s": "k_half_pc4<1>"}
 
 # algorithmic bytes per interior cell for one launch of each probed kernel (FP64):
