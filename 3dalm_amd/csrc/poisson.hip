@@ -906,7 +906,10 @@ static bool halves_pay(const dalm_ctx* ctx, const HalfGeom& G) {
 
 // Its split of a grid: every number of j tiles is priced, a block (one per compute unit:
 // its wavefronts fill the VGPRs) taking ni + 2 kFLag steps priced at 1.5 us + 0.3 us per
-// wavefront; no split where fewer than 10 rows fit a block (rows above 304 cells).
+// wavefront; no split where fewer than 8 rows fit a block (rows above 384 cells).  Half the rows
+// are halo then, and the halves are the faster kernels all the same: a step of 16 iterations
+// with the separate kernels and fused 7444 and 6337 us at 128x128x349, 7881 and 6670 at
+// 128x128x383, 28173 and 19833 at 256x200x383.
 HalfGeom split_pc(const dalm_ctx* ctx) {
     const Dims& d = ctx->d;
     const int Q = (d.nz + 3) / 4, most = kPcThreads / Q;
