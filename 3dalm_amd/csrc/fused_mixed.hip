@@ -546,8 +546,9 @@ HalfGeom split_half(const dalm_ctx* ctx) {
     return best;
 }
 
-// The fused path: three Jacobi sweeps on a grid that splits (R > 0).  It is the faster one
-// at every size measured, a step of 10 iterations with the separate kernels and fused:
+// The fused path: three Jacobi sweeps on a grid that splits (R > 0).  Of 240 sizes from 200 to
+// 5 10^6 cells it is the faster one at all but three (rows of 160 to 290 cells on grids of few
+// rows: at most 4 % slower, 661 and 685 us at 11x18x288): a step of 10 iterations with the separate kernels and fused:
 // 654 and 569 us at 30x14x16, 678 and 629 at 96x48x48, 806 and 701 at 128x64x64, 939 and 862 at
 // 64x96x128, 1295 and 1048 at 173x101x87, 8110 and 6366 at
 // 400x200x190, and of 12 iterations 2245 and 2058 at 256x128x128.  Rows too long for a
