@@ -100,13 +100,16 @@ def test_flux_rhs_bc(mesh, ok):
     assert np.array_equal(c.download("b"), b)
 
 
-def test_operator_and_sor(mesh, ok):
+# in one launch, as these grids are small, and with a launch per sweep
+@pytest.mark.parametrize("off", [(), ("one_launch",)])
+def test_operator_and_sor(mesh, ok, off):
     g = po.make_grid(mesh)
     A = np.zeros((mesh.L, 7))
     md = ok.build_A(g, A)
     p0 = rand_field(mesh, 11, 1, 0.1)
     b = rand_field(mesh, 12, 1, 1.0) * interior_mask(mesh)
     c = ctx_with(mesh, p=p0, b=b)
+    c.set_paths(off)
     assert c.build_A() == md
     r_ref = np.zeros(mesh.L)
     ok.residual(g, A, p0, b, r_ref)
@@ -125,14 +128,16 @@ def test_operator_and_sor(mesh, ok):
     assert abs(gerr - err.value) <= 1e-13 * err.value
 
 
+@pytest.mark.parametrize("off, on", [((), ()), (("one_launch",), ("halves",)), (("one_launch", "halves"), ())])
 @pytest.mark.parametrize("pc", [hip.PC_JACOBI, hip.PC_SOR])
-def test_bicgstab(mesh, ok, pc):
+def test_bicgstab(mesh, ok, pc, off, on):
     g = po.make_grid(mesh)
     A = np.zeros((mesh.L, 7))
     ok.build_A(g, A)
     p0 = rand_field(mesh, 21, 1, 0.1)
     b = rand_field(mesh, 22, 1, 1.0) * interior_mask(mesh)
     c = ctx_with(mesh, p=p0, b=b)
+    c.set_paths(off, on)
     x = p0.copy()
     work = np.zeros(9 * mesh.L)
     it, err = po.C.c_int64(), po.C.c_double()
@@ -173,6 +178,7 @@ def test_bicgstab_rows256_first_iterations(ok, shape, iters):
     p0 = rand_field(mesh, 31, 1, 0.1)
     b = rand_field(mesh, 32, 1, 1.0) * interior_mask(mesh)
     c = ctx_with(mesh, p=p0, b=b)
+    c.set_paths(("one_launch",))
     x = p0.copy()
     work = np.zeros(9 * mesh.L)
     it, err = po.C.c_int64(), po.C.c_double()
@@ -181,6 +187,7 @@ def test_bicgstab_rows256_first_iterations(ok, shape, iters):
     git, gerr, st = c.run_bicgstab(hip.PC_JACOBI, 1.0, 3, iters, 1e-30)
     print(f"bicgstab rows256, {iters} iterations: err {gerr:.6e} vs {err.value:.6e}", flush=True)
     assert git == it.value == iters and st == hip.NONCONVERGED
+    assert c.paths_taken()["halves" if shape == (40, 20, 256) else "launches"] == 1
     # the summation order's rounding grows with the iterations (allowed 10x per
     # iteration past the second); a pressure update left out would be off by far more
     grow = 10.0 ** (iters - 2)
